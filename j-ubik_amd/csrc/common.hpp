@@ -195,6 +195,23 @@ struct Tile {
   static constexpr int V = tile_vectors(JUBIK_COL_TILE_BYTES, L, (int)sizeof(cplx<T>));
 };
 
+// Column passes of the PSF operator: a tile of 128 bytes of every spectrum
+// row (one cache line: 16 float or 8 double columns), at most the L/2 stored
+// columns, whatever its length.  A half line per row is slower even where it
+// lets more work-groups share a CU (FP32, L = 432 in fold mode at 1024^2 x 4E,
+// forward / adjoint: 8 columns 186 / 168, 16 columns 162 / 140 us).  Two lines
+// pay at L = 192 in FP64 only, whose one-line work-group would be two waves
+// that the LDS keeps few of (512^2 x 4E: 42 / 39 against 37 / 35 us).
+__host__ __device__ constexpr int col_vectors(int L, int elem) {
+  int v = elem == 16 && L == 192 ? 16 : 128 / elem;
+  while (v > 8 && v / 2 >= L / 2) v /= 2;
+  return v;
+}
+template <typename T, int L>
+struct ColTile {
+  static constexpr int V = col_vectors(L, (int)sizeof(cplx<T>));
+};
+
 // Row passes use a quarter of that LDS budget: their global traffic is
 // contiguous rows whatever V is, and the smaller footprint raises residency
 // (at L = 384, 4 vectors per tile measured faster than 8 or 16).

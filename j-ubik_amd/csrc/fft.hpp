@@ -388,6 +388,50 @@ __host__ __device__ constexpr int lds_stride(int L, int V) {
   return L + ((r - L % 16) % 16 + 16) % 16;
 }
 
+// Threads per work-group of a pass over V vectors of length L that keeps
+// every value in registers from stage to stage (plan kind 0): the multiple of
+// 64 whose stages issue the fewest butterfly points, idle lanes counted, with
+// at most max_points values per thread and stage; among equals the one that
+// holds fewer values.
+__host__ __device__ constexpr int stage_points(int L, int V, int nt, int s) {
+  const int R = plan_radix(L, s);
+  return ((V * (L / R) + nt - 1) / nt) * R;
+}
+__host__ __device__ constexpr int register_threads(int L, int V, int max_points) {
+  for (int most_nt = 256; most_nt <= 512; most_nt += 256) {
+    int best = 0, best_cost = 0, best_most = 0;
+    for (int nt = 64; nt <= most_nt; nt += 64) {
+      int cost = 0, most = 0, radix = 0;
+      for (int s = 0; s < plan_stages(L); ++s) {
+        const int q = stage_points(L, V, nt, s);
+        cost += q * nt;
+        most = q > most ? q : most;
+        radix = plan_radix(L, s) > radix ? plan_radix(L, s) : radix;
+      }
+      if (most > max_points && most > radix) continue;
+      if (best == 0 || cost < best_cost || (cost == best_cost && most < best_most)) {
+        best = nt;
+        best_cost = cost;
+        best_most = most;
+      }
+    }
+    if (best > 0) return best;
+  }
+  return 512;
+}
+
+// LDS stride, in words of one real component, for exchanges of the real and
+// the imaginary parts one after the other (exchange_split): V vectors
+// interleaved over 64 (float) or 32 (double) bank slots.  The lanes of a wave
+// then meet the slots evenly both for consecutive positions (gathers) and
+// for positions a multiple of 16 apart (scatters of a radix-16 first stage).
+__host__ __device__ constexpr int split_stride(int L, int V, int elem) {
+  const int slots = 256 / elem;
+  const int per = slots / V > 8 ? slots / V : 8;
+  const int r = (V >= 16 ? 16 : per) + 1;
+  return L + ((r - L % slots) % slots + slots) % slots;
+}
+
 // ---------------------------------------------------------------- stages
 template <typename T, int L, bool INV, int S, int V, int VS, int NT, int PL = 0>
 struct Stage {
@@ -459,6 +503,34 @@ struct Stage {
       }
     }
   }
+  // One component (IM: imaginary) of gather_lds and scatter_lds, through a
+  // buffer of reals at vector stride VS.
+  template <bool IM>
+  static __device__ __forceinline__ void gather_part(const T* buf, Regs& v, int tid) {
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) {
+      int vec, j;
+      if (task(tid, b, vec, j)) {
+        const T* src = buf + vec * VS;
+#pragma unroll
+        for (int t = 0; t < R; ++t) (IM ? v[b][t].im : v[b][t].re) = src[j + t * NB];
+      }
+    }
+  }
+  template <bool IM>
+  static __device__ __forceinline__ void scatter_part(T* buf, const Regs& v, int tid) {
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) {
+      int vec, j;
+      if (task(tid, b, vec, j)) {
+        const int k = j % Ns;
+        T* dst = buf + vec * VS;
+        const int p0 = (j - k) * R + k;
+#pragma unroll
+        for (int t = 0; t < R; ++t) dst[p0 + t * Ns] = IM ? v[b][t].im : v[b][t].re;
+      }
+    }
+  }
   // Last stage only (Ns * R == L): dst(vec, j + t * NB, value).
   template <class Dst>
   static __device__ __forceinline__ void emit(const Regs& v, int tid, Dst dst) {
@@ -486,6 +558,32 @@ struct Stage {
     }
   }
 };
+
+// The outputs of stage A handed to the lanes that run stage B, as complex
+// values (T-typed buffer of 2 V VS reals).  Every lane must be past its last
+// read of ``buf`` on entry; reads are pending on exit.
+template <class A, class B, typename T>
+__device__ __forceinline__ void exchange_full(T* buf, const typename A::Regs& a,
+                                              typename B::Regs& b, int tid) {
+  cplx<T>* c = reinterpret_cast<cplx<T>*>(buf);
+  A::scatter_lds(c, a, tid);
+  __syncthreads();
+  B::gather_lds(c, b, tid);
+}
+
+// The same, real parts first: the tile needs half the LDS, which lets more
+// work-groups share a CU.
+template <class A, class B, typename T>
+__device__ __forceinline__ void exchange_split(T* buf, const typename A::Regs& a,
+                                               typename B::Regs& b, int tid) {
+  A::template scatter_part<false>(buf, a, tid);
+  __syncthreads();
+  B::template gather_part<false>(buf, b, tid);
+  __syncthreads();
+  A::template scatter_part<true>(buf, a, tid);
+  __syncthreads();
+  B::template gather_part<true>(buf, b, tid);
+}
 
 // Stages S..end, LDS -> LDS (a barrier after every scatter).
 template <typename T, int L, bool INV, int S, int V, int VS, int NT, int PL = 0>

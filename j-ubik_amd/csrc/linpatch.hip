@@ -44,7 +44,7 @@ int linpatch_fft_length(int w, int m) {
 int linpatch_col_tile(int dtype, int L, int col_div) {
   if ((dtype != 0 && dtype != 1) || !linpatch_length_supported(L)) return 0;
   if (col_div != 1 && col_div != 2 && col_div != 4) return 0;
-  const int v = tile_vectors(JUBIK_COL_TILE_BYTES, L, dtype == 0 ? 8 : 16) / col_div;
+  const int v = col_vectors(L, dtype == 0 ? 8 : 16) / col_div;
   return (col_div == 1 || v >= 2) ? v : 0;
 }
 

@@ -255,21 +255,7 @@ __global__ __launch_bounds__(NT) void lp_rows(LinGeom g, const T* __restrict__ s
 // ------------------------------------------------------------------ cols
 // Forward stages, then (signal modes) the spectrum multiply and the inverse
 // stages; the last forward and first inverse stage share registers.
-template <typename T, int L, bool INV, int S, int V, int VS, int NT_>
-__device__ __forceinline__ void stages_mid(cplx<T>* buf, const cplx<T>* tw, int tid) {
-  // stages S .. plan_stages(L) - 2 (all but the last), LDS -> LDS
-  if constexpr (S + 1 < plan_stages(L)) {
-    using St = Stage<T, L, INV, S, V, VS, NT_>;
-    typename St::Regs v;
-    St::gather_lds(buf, v, tid);
-    St::compute(v, tw, tid);
-    __syncthreads();
-    St::scatter_lds(buf, v, tid);
-    __syncthreads();
-    stages_mid<T, L, INV, S + 1, V, VS, NT_>(buf, tw, tid);
-  }
-}
-
+//
 // Exchange the forward spectrum of the packed column (tile 0, vector 0)
 // through LDS so each position can read its mirror P[-f].  Called by the
 // whole work-group once every thread has finished reading buf.
@@ -281,6 +267,34 @@ __device__ __forceinline__ void share_packed(cplx<T>* buf, typename FL::Regs& la
   });
   __syncthreads();
 }
+
+// Threads per work-group of the column pass over V columns (register_threads):
+// at most 32 values per thread in FP32; in FP64 one butterfly per thread.
+// With 256 threads whatever the length, a stage of L/R butterflies per column
+// that do not divide by 256 gave some threads two butterflies' registers and
+// left the others idle: at L = 324 (18 x 18, 288 butterflies of 18 points)
+// 177 VGPRs and 2 waves per SIMD against 96 and 5 at 320 threads; in FP64 most
+// lengths ran half empty (measured at 1024^2 x 4E, L = 432 in fold mode,
+// forward / adjoint: 448 / 414 -> 301 / 272 us; L = 512: 603 / 617 -> 328 /
+// 329 us; L = 320 at 512^2: 43 / 43 -> 36 / 33 us).
+template <typename T, int L, int V>
+struct ColThreads {
+  static constexpr int NT = register_threads(L, V, sizeof(T) == 4 ? 32 : 0);
+};
+
+// Exchanges between the stages: complex values, or one component at a time
+// (exchange_split) in FP32 at L = 192, 324 and 432, where the complex tile's
+// LDS and not the registers would bound the resident work-groups.  Measured
+// at 1024^2 x 4E, forward / adjoint, complex against split: L = 324 127 / 108
+// against 107 / 91 us, L = 432 (fold mode) 205 / 162 against 162 / 140 us,
+// L = 192 at 512^2 x 3E 22 / 20 against 17.5 / 16.7 us; elsewhere the two
+// barriers more cost as much as they give (L = 384 82 / 65 against 84 / 67 us,
+// L = 512 133 / 122 against 138 / 127 us, L = 224 at 768^2 52 / 42 against
+// 53 / 43 us, FP64 equal).
+template <typename T, int L>
+struct ColSplit {
+  static constexpr bool value = sizeof(T) == 4 && (L == 192 || L == 324 || L == 432);
+};
 
 // 1-D grid over (sample, column tile, patch, z) with the sample fastest;
 // z < M * Ek spectra (kernel mode) or J jobs per sample.  Work-groups are
@@ -301,18 +315,22 @@ __device__ __forceinline__ void share_packed(cplx<T>* buf, typename FL::Regs& la
 // grid order below) and meet them in its L2.  The forward multiplies each
 // window row by its tent weight on load, through a zero-reading gather so
 // that the multiply does not pull each load into a branch of its own.
-template <typename T, int L, int MODE, int VC = Tile<T, L>::V, bool FOLD = false>
-__global__ __launch_bounds__(NT) void lp_cols(LinGeom g, const cplx<T>* __restrict__ R1,
+template <typename T, int L, int MODE, int VC = ColTile<T, L>::V, bool FOLD = false>
+__global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g, const cplx<T>* __restrict__ R1,
                                               const cplx<T>* __restrict__ KT,
                                               const cplx<T>* __restrict__ twg,
                                               cplx<T>* __restrict__ out,
                                               cplx<T>* __restrict__ KB, NllFinal fin) {
   constexpr int V = VC;
-  constexpr int VS = lds_stride(L, V);
+  constexpr int NT = ColThreads<T, L, VC>::NT;
+  constexpr bool SPLIT = ColSplit<T, L>::value;
+  constexpr int VS = SPLIT ? split_stride(L, V, (int)sizeof(T)) : lds_stride(L, V);
   constexpr int LH = L / 2;
   constexpr int L2P = half_stride(L);
   constexpr int NS = plan_stages(L);
-  __shared__ cplx<T> buf[V * VS];
+  static_assert(NS <= 2, "the column pass runs plans of one or two stages");
+  static_assert(V >= 2, "the exchange buffer also holds one complex column");
+  __shared__ __align__(16) T buf[(SPLIT ? 1 : 2) * V * VS];
   __shared__ cplx<T> tw[L];
   __shared__ double red[NT / 64];
   __shared__ double total_s;
@@ -432,14 +450,15 @@ __global__ __launch_bounds__(NT) void lp_cols(LinGeom g, const cplx<T>* __restri
     store_twiddles();
     tent_rows(v0);
     F0::compute(v0, tw, tid);
-    F0::scatter_lds(buf, v0, tid);
-    __syncthreads();
-    stages_mid<T, L, false, 1, V, VS, NT>(buf, tw, tid);
-    FL::gather_lds(buf, last, tid);
+    if constexpr (SPLIT)
+      exchange_split<F0, FL>(buf, v0, last, tid);
+    else
+      exchange_full<F0, FL>(buf, v0, last, tid);
     FL::compute(last, tw, tid);
   }
 
-  if (k0 == 0) share_packed<FL, T, L>(buf, last, tid);
+  cplx<T>* packed = reinterpret_cast<cplx<T>*>(buf);
+  if (k0 == 0) share_packed<FL, T, L>(packed, last, tid);
   if constexpr (MODE == COL_KERNEL) {
     cplx<T>* kt = out + spec * L2P * L;
     FL::emit(last, tid, [&](int vec, int pos, cplx<T> val) {
@@ -448,7 +467,7 @@ __global__ __launch_bounds__(NT) void lp_cols(LinGeom g, const cplx<T>* __restri
       if (k == 0) {
         // K0 = (P + conj P-)/2, KN = (P - conj P-)/(2i), each with its
         // ifftshift sign (-1)^(f + k) and the normalisation.
-        const cplx<T> pm = buf[pos == 0 ? 0 : L - pos];
+        const cplx<T> pm = packed[pos == 0 ? 0 : L - pos];
         const T s0 = (pos & 1) ? -factor : factor;
         const T sn = ((pos + LH) & 1) ? -factor : factor;
         const cplx<T> k0v = {T(0.5) * s0 * (val.re + pm.re), T(0.5) * s0 * (val.im - pm.im)};
@@ -477,7 +496,7 @@ __global__ __launch_bounds__(NT) void lp_cols(LinGeom g, const cplx<T>* __restri
 #pragma unroll
           for (int t = 0; t < FL::R; ++t) {
             const int pos = j + t * FL::NB;
-            const cplx<T> pm = buf[pos == 0 ? 0 : L - pos];
+            const cplx<T> pm = packed[pos == 0 ? 0 : L - pos];
             const cplx<T> pc = {pm.re, -pm.im};
             const cplx<T> be = KB[spec * L + pos];
             last[b][t] = cadd(last[b][t], (MODE == COL_ADJ) ? cmulc(pc, be) : cmul(pc, be));
@@ -503,51 +522,63 @@ __global__ __launch_bounds__(NT) void lp_cols(LinGeom g, const cplx<T>* __restri
         if (ir >= 0 && ir < g.H) st_stream(&o[pos * L2P + k], val);
       }
     };
-    // Fold mode, forward: the transformed columns go to LDS, and output row
-    // q of the Lw window sums frame positions c, c + Lw and c - Lw, c = q +
-    // mf - m (in [0, L) because L >= Lw); rows outside the image are skipped
-    // as above.
-    auto to_lds = [&](int vec, int pos, cplx<T> val) { buf[vec * VS + pos] = val; };
-    auto fold_out = [&]() {
-      __syncthreads();
+    // Fold mode, forward: the transformed columns go to LDS, one component
+    // after the other, and output row q of the Lw window sums frame positions
+    // c, c + Lw and c - Lw, c = q + mf - m (in [0, L) because L >= Lw); rows
+    // outside the image are skipped as above.
+    constexpr bool kFoldOut = FOLD && MODE == COL_FWD;
+    constexpr int FPT = kFoldOut ? (V * L + NT - 1) / NT : 1;
+    auto fold_part = [&](T (&sum)[FPT]) {
       const int off = g.mf - g.m;
-      for (int e = tid; e < V * lw; e += NT) {
-        const int vec = e & (V - 1), q = e / V;
-        const int k = k0 + vec;
-        const int ir = row0 + q;
-        if (k >= LH || ir < 0 || ir >= g.H) continue;
-        const int c = q + off;
-        const cplx<T>* col = buf + vec * VS;
-        cplx<T> acc = col[c];
-        if (c + lw < L) acc = cadd(acc, col[c + lw]);
-        if (c >= lw) acc = cadd(acc, col[c - lw]);
-        st_stream(&o[q * L2P + k], acc);
+#pragma unroll
+      for (int u = 0; u < FPT; ++u) {
+        const int e = tid + u * NT;
+        if (e >= V * lw) break;
+        const int c = e / V + off;
+        const T* col = buf + (e & (V - 1)) * VS;
+        T acc = col[c];
+        if (c + lw < L) acc += col[c + lw];
+        if (c >= lw) acc += col[c - lw];
+        sum[u] = acc;
       }
     };
-    constexpr bool kFoldOut = FOLD && MODE == COL_FWD;
+    auto fold_out = [&](auto stage, auto& vals) {
+      using St = decltype(stage);
+      T re[FPT], im[FPT];
+      __syncthreads();
+      St::emit(vals, tid, [&](int vec, int pos, cplx<T> val) { buf[vec * VS + pos] = val.re; });
+      __syncthreads();
+      fold_part(re);
+      __syncthreads();
+      St::emit(vals, tid, [&](int vec, int pos, cplx<T> val) { buf[vec * VS + pos] = val.im; });
+      __syncthreads();
+      fold_part(im);
+#pragma unroll
+      for (int u = 0; u < FPT; ++u) {
+        const int e = tid + u * NT;
+        if (e >= V * lw) break;
+        const int k = k0 + (e & (V - 1)), q = e / V;
+        const int ir = row0 + q;
+        if (k < LH && ir >= 0 && ir < g.H) st_stream(&o[q * L2P + k], cplx<T>{re[u], im[u]});
+      }
+    };
     if constexpr (NS == 1) {
-      if constexpr (kFoldOut) {
-        __syncthreads();
-        I0::emit(last, tid, to_lds);
-        fold_out();
-      } else {
+      if constexpr (kFoldOut)
+        fold_out(I0{}, last);
+      else
         I0::emit(last, tid, store);
-      }
     } else {
-      __syncthreads();
-      I0::scatter_lds(buf, last, tid);
-      __syncthreads();
-      stages_mid<T, L, true, 1, V, VS, NT>(buf, tw, tid);
       typename IL::Regs v;
-      IL::gather_lds(buf, v, tid);
+      __syncthreads();
+      if constexpr (SPLIT)
+        exchange_split<I0, IL>(buf, last, v, tid);
+      else
+        exchange_full<I0, IL>(buf, last, v, tid);
       IL::compute(v, tw, tid);
-      if constexpr (kFoldOut) {
-        __syncthreads();
-        IL::emit(v, tid, to_lds);
-        fold_out();
-      } else {
+      if constexpr (kFoldOut)
+        fold_out(IL{}, v);
+      else
         IL::emit(v, tid, store);
-      }
     }
   }
   if constexpr (MODE == COL_ADJ) {
@@ -1078,8 +1109,10 @@ static int launch_status(const char* what) {
 
 template <typename T, int L>
 struct LinOps {
-  static constexpr int V = Tile<T, L>::V;
+  static constexpr int V = ColTile<T, L>::V;
   static constexpr int VR = RowTile<T, L>::V;
+  template <int VC>
+  static constexpr int kColThreads = ColThreads<T, L, VC>::NT;
   static constexpr int LH = L / 2;
   using C = cplx<T>;
 
@@ -1101,7 +1134,7 @@ struct LinOps {
     const int gc = (LH + V - 1) / V * g.P * g.M * g.Ek;
     {
       TimedLaunch _t("lp_cols_kernel", s);
-      lp_cols<T, L, COL_KERNEL><<<gc, NT, 0, s>>>(g, (const C*)b.R1, nullptr, (const C*)b.tw,
+      lp_cols<T, L, COL_KERNEL><<<gc, kColThreads<V>, 0, s>>>(g, (const C*)b.R1, nullptr, (const C*)b.tw,
                                                   (C*)b.KT, (C*)b.KB, NllFinal{});
     }
     return launch_status("linpatch_prepare");
@@ -1139,7 +1172,7 @@ struct LinOps {
       with_cols(g, b, [&](auto vc) {
         constexpr int VC = decltype(vc)::value;
         const int gc = g.S * ((LH + VC - 1) / VC) * g.P * g.J;
-        lp_cols<T, L, COL_FWD, VC, FOLD><<<gc, NT, 0, s>>>(g, (const C*)b.R1, (const C*)b.KT,
+        lp_cols<T, L, COL_FWD, VC, FOLD><<<gc, kColThreads<VC>, 0, s>>>(g, (const C*)b.R1, (const C*)b.KT,
                                                            (const C*)b.tw, (C*)b.R2, (C*)b.KB,
                                                            NllFinal{});
       });
@@ -1171,7 +1204,7 @@ struct LinOps {
       with_cols(g, b, [&](auto vc) {
         constexpr int VC = decltype(vc)::value;
         const int gc = g.S * ((LH + VC - 1) / VC) * g.P * g.J;
-        lp_cols<T, L, COL_ADJ, VC, FOLD><<<gc, NT, 0, s>>>(g, (const C*)b.R1, (const C*)b.KT,
+        lp_cols<T, L, COL_ADJ, VC, FOLD><<<gc, kColThreads<VC>, 0, s>>>(g, (const C*)b.R1, (const C*)b.KT,
                                                            (const C*)b.tw, (C*)b.R2, (C*)b.KB,
                                                            fin);
       });
