@@ -298,6 +298,12 @@ int jubik_model_metric(jubik_model* model, const void* amp_ref, const void* amp_
  * counts[0 .. S) when counts is not NULL and returns JUBIK_EDOMAIN with a
  * message when any is positive. */
 int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream);
+/* The last gradient evaluation's results without a device-to-host copy: the
+ * kernels write the S NLL values and the counts of the domain check to
+ * page-locked host memory of the model, too.  Synchronises ``stream``, writes
+ * nll[0 .. S) and counts[0 .. S) (each may be NULL) and returns JUBIK_EDOMAIN
+ * as jubik_model_check_domain does. */
+int jubik_model_result(jubik_model* model, double* nll, int64_t* counts, void* stream);
 /* S gradient evaluations in one pass: xi_ref, xi_alpha, g_ref, g_alpha are
  * (S, N, N) stacks, nll holds S device doubles.  The metric base point is
  * not changed. */

@@ -43,6 +43,9 @@ def code(dtype):
 def to_device(a, dtype):
     """Contiguous device tensor of ``dtype`` holding ``a``."""
     if isinstance(a, torch.Tensor):
+        if (a.is_cuda and a.dtype == dtype and a.get_device() == torch.cuda.current_device()
+                and a.is_contiguous()):
+            return a
         t = a.to(device="cuda", dtype=dtype)
     else:
         t = torch.as_tensor(np.asarray(a), dtype=dtype, device="cuda")

@@ -63,6 +63,7 @@ SIGNATURES = {
                                _vp, _vp],
     "jubik_model_metric": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "jubik_model_check_domain": [_vp, _vp, _vp],
+    "jubik_model_result": [_vp, _dblp, _vp, _vp],
     "jubik_linpatch_set_tile": [_vp, _int, _int],
     "jubik_linpatch_set_transform": [_vp, _int],
     "jubik_linpatch_autotune": [_vp, _int, C.POINTER(_int), C.POINTER(_int), _dblp, _vp],
@@ -149,7 +150,7 @@ def check(status):
 
 
 def call(name, *args):
-    check(getattr(load(), name)(*args))
+    check(getattr(_lib or load(), name)(*args))
 
 
 def timing_enable(on=True):

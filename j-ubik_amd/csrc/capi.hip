@@ -93,6 +93,22 @@ int dev_alloc(void** p, size_t bytes, const char* what) {
   return kOk;
 }
 
+// Page-locked host memory that kernels write through (NllFinal::report).
+int host_alloc(void** p, size_t bytes, const char* what) {
+  *p = nullptr;
+  if (g_fail_alloc.load() > 0 && g_fail_alloc.fetch_sub(1) == 1)
+    return fail(kOutOfMemory, std::string("allocating ") + what + ": injected failure");
+  hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+    return fail(e == hipErrorOutOfMemory ? kOutOfMemory : kRuntimeError,
+                std::string("allocating ") + what + " (" + std::to_string(bytes) +
+                    " bytes): " + hipGetErrorString(e));
+  }
+  return kOk;
+}
+
 void dev_free(void*& p) {
   if (p) (void)hipFree(p);
   p = nullptr;
@@ -209,7 +225,7 @@ struct jubik_model {
   void* dsky = nullptr;     // max_samples x E x H x W
   void* resid = nullptr;    // max_samples x J x H x W
   void* partial = nullptr;  // 2 x max_samples x J x H doubles (NLL terms, lam <= 0 counts)
-  void* nbad = nullptr;     // max_samples doubles: read-out pixels with lam <= 0
+  void* report = nullptr;   // host, 2 x max_samples doubles: NLL and lam <= 0 counts
   int last_S = 0;           // samples of the last gradient evaluation
   int batch_S = 0;          // samples of the last batched gradient (slots 1 .. S)
   void* cg_vec = nullptr;   // solver vectors r, p, Ap, Mv: 4 x max_samples x 2 x N^2
@@ -244,7 +260,8 @@ struct jubik_model {
     dev_free(resid);
     dev_free(lam);
     dev_free(partial);
-    dev_free(nbad);
+    if (report) (void)hipHostFree(report);
+    report = nullptr;
     dev_free(cg_vec);
     dev_free(cg_work);
     dev_free(u);
@@ -959,7 +976,7 @@ int jubik_model_create_batched(jubik_model** model, jubik_gp* gp, jubik_linpatch
   if (!st) st = dev_alloc(&m->dsky, img * g.E * S * es, "sky tangent");
   if (!st) st = dev_alloc(&m->resid, img * g.J * S * es, "residual");
   if (!st) st = dev_alloc(&m->partial, 2 * (size_t)g.J * g.H * S * sizeof(double), "NLL partials");
-  if (!st) st = dev_alloc(&m->nbad, S * sizeof(double), "lambda domain counts");
+  if (!st) st = host_alloc(&m->report, 2 * S * sizeof(double), "evaluation report");
   // GP cotangent: E real planes per sample, or one complex plane (energies
   // folded in) per sample
   if (!st) st = dev_alloc(&m->u, img * std::max(g.E, 2) * S * es, "GP cotangent planes");
@@ -1050,7 +1067,8 @@ int model_grad(jubik_model* model, int S, int slot0, const void* amp_ref, const 
   fin.seglen = (int64_t)g.J * g.H;
   fin.nseg = S;
   fin.out = nll;
-  fin.bad_out = (double*)model->nbad;
+  fin.report = (double*)model->report;
+  fin.report_n = model->max_samples;
   model->last_S = S;
   if (slot0 == 1) model->batch_S = S;
   st = linpatch_adjoint_gp(lp->dtype, g, model->lbufs(), model->resid, model->pixel_area, sky,
@@ -1771,20 +1789,19 @@ int jubik_model_metric(jubik_model* model, const void* amp_ref, const void* amp_
                                   out_alpha, stream);
 }
 
-int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream) {
+int jubik_model_result(jubik_model* model, double* nll, int64_t* counts, void* stream) {
   if (!model) return fail(kInvalidArgument, "NULL argument");
   if (model->last_S < 1) return fail(kNotReady, "no gradient evaluation yet");
   DeviceGuard dg(model->lp->device);
-  std::vector<double> nb(model->last_S);
-  hipStream_t s = as_stream(stream);
-  JUBIK_HIP(hipMemcpyAsync(nb.data(), model->nbad, nb.size() * sizeof(double),
-                           hipMemcpyDeviceToHost, s));
-  JUBIK_HIP(hipStreamSynchronize(s));
+  JUBIK_HIP(hipStreamSynchronize(as_stream(stream)));
+  const double* rep = static_cast<const double*>(model->report);
   std::string bad;
-  for (size_t k = 0; k < nb.size(); ++k) {
-    if (counts) counts[k] = (int64_t)nb[k];
-    if (nb[k] > 0)
-      bad += (bad.empty() ? "" : ", ") + std::to_string((int64_t)nb[k]) + " at sample " +
+  for (int k = 0; k < model->last_S; ++k) {
+    const double nb = rep[model->max_samples + k];
+    if (nll) nll[k] = rep[k];
+    if (counts) counts[k] = (int64_t)nb;
+    if (nb > 0)
+      bad += (bad.empty() ? "" : ", ") + std::to_string((int64_t)nb) + " at sample " +
              std::to_string(k);
   }
   if (!bad.empty())
@@ -1792,6 +1809,10 @@ int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream) 
                              "): the Poisson NLL is inf or NaN there; mask pixels with zero "
                              "exposure");
   return kOk;
+}
+
+int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream) {
+  return jubik_model_result(model, nullptr, counts, stream);
 }
 
 int jubik_graph_capture_metric_batch(jubik_graph** out, const jubik_metric_desc* descs,

@@ -72,14 +72,17 @@ int linpatch_adjoint(int dtype, const LinGeom& g, const LinBuffers& b, const voi
 // NLL finalisation folded into the adjoint column pass, which starts after
 // the forward has written every partial: out[b] = sum of partial[b * seglen
 // .. (b + 1) * seglen) for b < nseg, in a fixed order (no extra launch).
-// With bad_out set, bad_out[b] also receives the count of read-out pixels
-// with lam <= 0 of segment b (stored nseg * seglen after the NLL terms).
+// report: page-locked host memory that the kernel writes through, so the
+// caller reads the results after one stream synchronisation and no copy:
+// report[b] = out[b], report[report_n + b] = count of read-out pixels with lam
+// <= 0 of segment b (stored nseg * seglen after the NLL terms).
 struct NllFinal {
   const double* partial = nullptr;
   int64_t seglen = 0;
   int nseg = 0;
   double* out = nullptr;
-  double* bad_out = nullptr;
+  double* report = nullptr;
+  int report_n = 0;
 };
 
 // Adjoint chained into the GP, with v_(s,e) = sum_mod scale * sky[e] *

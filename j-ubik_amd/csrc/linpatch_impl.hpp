@@ -589,14 +589,17 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
       double acc = 0.0, nb = 0.0;
       for (int64_t k = tid; k < fin.seglen; k += NT) acc += pp[k];
       acc = block_sum<NT>(acc, red);
-      if (fin.bad_out) {
+      if (fin.report) {
         const double* pb = pp + (int64_t)fin.nseg * fin.seglen;
         for (int64_t k = tid; k < fin.seglen; k += NT) nb += pb[k];
         nb = block_sum<NT>(nb, red);
       }
       if (tid == 0) {
         fin.out[blockIdx.x] = acc;
-        if (fin.bad_out) fin.bad_out[blockIdx.x] = nb;
+        if (fin.report) {
+          fin.report[blockIdx.x] = acc;
+          fin.report[fin.report_n + blockIdx.x] = nb;
+        }
       }
     }
   }

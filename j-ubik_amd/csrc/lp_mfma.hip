@@ -221,14 +221,17 @@ __global__ __launch_bounds__(MNT) void lp_cols_mfma(LinGeom g, const bf16x8* __r
       double acc = 0.0, nb = 0.0;
       for (int64_t k = tid; k < fin.seglen; k += MNT) acc += pp[k];
       acc = block_sum<MNT>(acc, red);
-      if (fin.bad_out) {
+      if (fin.report) {
         const double* pb = pp + (int64_t)fin.nseg * fin.seglen;
         for (int64_t k = tid; k < fin.seglen; k += MNT) nb += pb[k];
         nb = block_sum<MNT>(nb, red);
       }
       if (tid == 0) {
         fin.out[blockIdx.x] = acc;
-        if (fin.bad_out) fin.bad_out[blockIdx.x] = nb;
+        if (fin.report) {
+          fin.report[blockIdx.x] = acc;
+          fin.report[fin.report_n + blockIdx.x] = nb;
+        }
       }
     }
   }

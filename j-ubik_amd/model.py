@@ -184,14 +184,14 @@ class XrayModel:
                   dev.ptr(s.amp_alpha), dev.ptr(xr), dev.ptr(xa), s.zm, s.mu,
                   dev.ptr(s.dnu_dev), dev.ptr(xp), dev.ptr(xpa), dev.ptr(nll), dev.ptr(g_ref),
                   dev.ptr(g_alpha), dev.ptr(g_ps), dev.ptr(g_psa), dev.stream())
-        self.check_domain()
+        vals = self._result(S)
         if batch:
             self._batch_S = S
             self._batch_version = s.version
-            out_nll = nll.cpu().numpy()
+            out_nll = np.array(vals, dtype=np.float64)
         else:
             self._point_version = s.version
-            out_nll = float(nll.item())
+            out_nll = vals[0]
         like = lambda t: None if t is None else dev.like_input(t, xi_ps)
         return out_nll, like(g_ref), like(g_alpha), like(g_ps), like(g_psa)
 
@@ -208,12 +208,20 @@ class XrayModel:
             _lib.check(st)
         return counts
 
+    def _result(self, S=1):
+        """The S NLL values of the gradient evaluation just enqueued, after
+        one synchronisation with the stream (the kernels write them, with the
+        counts of ``check_domain``, to host memory).  Raises as
+        ``check_domain`` does."""
+        nll = (ctypes.c_double * S)()
+        _lib.call("jubik_model_result", self._model, nll, None, dev.stream())
+        return nll
+
     def nll_and_grad(self, xi_ref, xi_alpha=None):
         """(NLL as a Python float, grad_xi_ref, grad_xi_alpha).  Raises
         FloatingPointError when lam <= 0 at a read-out pixel."""
-        nll, g_ref, g_alpha = self.nll_and_grad_device(xi_ref, xi_alpha)
-        self.check_domain()
-        val = float(nll.item())
+        _, g_ref, g_alpha = self.nll_and_grad_device(xi_ref, xi_alpha)
+        val = self._result()[0]
         return val, dev.like_input(g_ref, xi_ref), (
             dev.like_input(g_alpha, xi_ref) if g_alpha is not None else None)
 
@@ -242,8 +250,7 @@ class XrayModel:
                   dev.ptr(s.dnu_dev), dev.ptr(self._nll), dev.ptr(g_ref), dev.ptr(g_alpha),
                   dev.ptr(ga_ref), dev.ptr(ga_alpha), dev.ptr(off), dev.stream())
         self._point_version = s.version
-        self.check_domain()
-        val = float(self._nll.item())
+        val = self._result()[0]
         offs = off.double().cpu().numpy()
         like = lambda t: None if t is None else dev.like_input(t, xi_ref)
         return (val, like(g_ref), like(g_alpha), like(ga_ref), like(ga_alpha), float(offs[0]),
@@ -289,10 +296,10 @@ class XrayModel:
         _lib.call("jubik_model_grad_batch", self._model, S, dev.ptr(s.amp_ref),
                   dev.ptr(s.amp_alpha), dev.ptr(xr), dev.ptr(xa), s.zm, s.mu, dev.ptr(s.dnu_dev),
                   dev.ptr(nll), dev.ptr(g_ref), dev.ptr(g_alpha), dev.stream())
-        self.check_domain()
+        vals = self._result(S)
         self._batch_S = S
         self._batch_version = s.version
-        return nll.cpu().numpy(), dev.like_input(g_ref, xi_ref), (
+        return np.array(vals, dtype=np.float64), dev.like_input(g_ref, xi_ref), (
             dev.like_input(g_alpha, xi_ref) if g_alpha is not None else None)
 
     def metric_batch(self, v_ref, v_alpha=None):
@@ -421,8 +428,7 @@ class XrayModel:
                   dev.ptr(s.amp_alpha), dev.ptr(xr), dev.ptr(xa), s.zm, s.mu,
                   dev.ptr(s.dnu_dev), dev.ptr(nll), dev.stream())
         self._batch_S = 0  # the batch slot now holds x
-        self.check_domain()
-        return float(nll.item())
+        return self._result()[0]
 
     def geovi_apply(self, mode, v_ref=None, v_alpha=None):
         """The geoVI operators at the base point p and the last geovi_point x:
