@@ -304,6 +304,20 @@ int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream);
  * nll[0 .. S) and counts[0 .. S) (each may be NULL) and returns JUBIK_EDOMAIN
  * as jubik_model_check_domain does. */
 int jubik_model_result(jubik_model* model, double* nll, int64_t* counts, void* stream);
+/* The sampled KL of optimize_kl (demos/x-ray-imaging.py:404-430) at the mean
+ * xbar (N x N) for S offsets delta (S x N x N): positions pos[s] = xbar +
+ * delta[s], the batched gradient at them (nll[s], gs[s]; they become the
+ * model's sample positions), and g = mean over s of gs[s] + pos[s], summed in
+ * double.  pos and gs are the caller's; the alpha arrays may be NULL without a
+ * spectral-index field.  Allocates nothing and does not synchronise. */
+int jubik_model_kl_grad(jubik_model* model, int64_t S, const void* amp_ref,
+                        const void* amp_alpha, const void* xbar_ref, const void* xbar_alpha,
+                        const void* delta_ref, const void* delta_alpha, double zm, double mu,
+                        const void* dnu, double* nll, void* pos_ref, void* pos_alpha,
+                        void* gs_ref, void* gs_alpha, void* g_ref, void* g_alpha, void* stream);
+/* jubik_model_result of the last jubik_model_kl_grad, with prior[0] = sum of
+ * all squared positions. */
+int jubik_model_kl_result(jubik_model* model, double* nll, double* prior, void* stream);
 /* S gradient evaluations in one pass: xi_ref, xi_alpha, g_ref, g_alpha are
  * (S, N, N) stacks, nll holds S device doubles.  The metric base point is
  * not changed. */

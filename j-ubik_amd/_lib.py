@@ -64,6 +64,9 @@ SIGNATURES = {
     "jubik_model_metric": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "jubik_model_check_domain": [_vp, _vp, _vp],
     "jubik_model_result": [_vp, _dblp, _vp, _vp],
+    "jubik_model_kl_grad": [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _dbl, _dbl, _vp, _vp, _vp,
+                            _vp, _vp, _vp, _vp, _vp, _vp],
+    "jubik_model_kl_result": [_vp, _dblp, _dblp, _vp],
     "jubik_linpatch_set_tile": [_vp, _int, _int],
     "jubik_linpatch_set_transform": [_vp, _int],
     "jubik_linpatch_autotune": [_vp, _int, C.POINTER(_int), C.POINTER(_int), _dblp, _vp],

@@ -11,6 +11,7 @@
 #include "../../include/jubik_hip.h"
 #include "cg.hpp"
 #include "gp.hpp"
+#include "kl.hpp"
 #include "points.hpp"
 #include "linpatch.hpp"
 #include "dft128.hpp"
@@ -225,7 +226,9 @@ struct jubik_model {
   void* dsky = nullptr;     // max_samples x E x H x W
   void* resid = nullptr;    // max_samples x J x H x W
   void* partial = nullptr;  // 2 x max_samples x J x H doubles (NLL terms, lam <= 0 counts)
-  void* report = nullptr;   // host, 2 x max_samples doubles: NLL and lam <= 0 counts
+  // host, 2 x max_samples + 1 doubles: NLL and lam <= 0 counts of the last
+  // evaluation, and the sum of squared positions of the last sampled KL
+  void* report = nullptr;
   int last_S = 0;           // samples of the last gradient evaluation
   int batch_S = 0;          // samples of the last batched gradient (slots 1 .. S)
   void* cg_vec = nullptr;   // solver vectors r, p, Ap, Mv: 4 x max_samples x 2 x N^2
@@ -976,7 +979,7 @@ int jubik_model_create_batched(jubik_model** model, jubik_gp* gp, jubik_linpatch
   if (!st) st = dev_alloc(&m->dsky, img * g.E * S * es, "sky tangent");
   if (!st) st = dev_alloc(&m->resid, img * g.J * S * es, "residual");
   if (!st) st = dev_alloc(&m->partial, 2 * (size_t)g.J * g.H * S * sizeof(double), "NLL partials");
-  if (!st) st = host_alloc(&m->report, 2 * S * sizeof(double), "evaluation report");
+  if (!st) st = host_alloc(&m->report, (2 * S + 1) * sizeof(double), "evaluation report");
   // GP cotangent: E real planes per sample, or one complex plane (energies
   // folded in) per sample
   if (!st) st = dev_alloc(&m->u, img * std::max(g.E, 2) * S * es, "GP cotangent planes");
@@ -1230,6 +1233,43 @@ int jubik_model_grad_batch(jubik_model* model, int64_t S, const void* amp_ref,
   DeviceGuard dg(model->lp->device);
   return model_grad(model, (int)S, 1, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll,
                     g_ref, g_alpha, as_stream(stream));
+}
+
+int jubik_model_kl_grad(jubik_model* model, int64_t S, const void* amp_ref,
+                        const void* amp_alpha, const void* xbar_ref, const void* xbar_alpha,
+                        const void* delta_ref, const void* delta_alpha, double zm, double mu,
+                        const void* dnu, double* nll, void* pos_ref, void* pos_alpha,
+                        void* gs_ref, void* gs_alpha, void* g_ref, void* g_alpha, void* stream) {
+  if (!model || !nll || !amp_ref || !xbar_ref || !delta_ref || !pos_ref || !gs_ref || !g_ref)
+    return fail(kInvalidArgument, "NULL argument");
+  if (S < 1 || S > model->max_samples)
+    return fail(kInvalidArgument, "batch of " + std::to_string(S) +
+                                      " samples outside [1, max_samples = " +
+                                      std::to_string(model->max_samples) + "]");
+  int st = check_model(model);
+  if (!st) st = check_alpha(model, amp_alpha, xbar_alpha, g_alpha, dnu);
+  if (!st) st = check_alpha(model, delta_alpha, pos_alpha, gs_alpha, dnu);
+  if (st) return st;
+  DeviceGuard dg(model->lp->device);
+  const int dtype = model->lp->dtype;
+  const bool alpha = model->gp->g.has_alpha != 0;
+  const int64_t n = (int64_t)model->gp->g.N * model->gp->g.N;
+  hipStream_t s = as_stream(stream);
+  KlFields f{{xbar_ref, alpha ? xbar_alpha : nullptr},
+             {delta_ref, delta_alpha},
+             {pos_ref, pos_alpha},
+             {gs_ref, gs_alpha},
+             {g_ref, g_alpha}};
+  // the partials of the prior energy borrow the NLL's, which the gradient
+  // fills only afterwards
+  const int64_t max_partial = 2LL * model->max_samples * model->lp->g.J * model->lp->g.H;
+  st = kl_positions(dtype, (int)S, n, f, (double*)model->partial, max_partial,
+                    (double*)model->report + 2 * model->max_samples, s);
+  if (!st)
+    st = model_grad(model, (int)S, 1, amp_ref, amp_alpha, pos_ref, pos_alpha, zm, mu, dnu, nll,
+                    gs_ref, gs_alpha, s);
+  if (!st) st = kl_mean(dtype, (int)S, n, f, s);
+  return st;
 }
 
 int jubik_model_set_tile(jubik_model* model, int col_div, int row_div) {
@@ -1809,6 +1849,12 @@ int jubik_model_result(jubik_model* model, double* nll, int64_t* counts, void* s
                              "): the Poisson NLL is inf or NaN there; mask pixels with zero "
                              "exposure");
   return kOk;
+}
+
+int jubik_model_kl_result(jubik_model* model, double* nll, double* prior, void* stream) {
+  const int st = jubik_model_result(model, nll, nullptr, stream);
+  if (!st && prior) *prior = static_cast<const double*>(model->report)[2 * model->max_samples];
+  return st;
 }
 
 int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream) {

@@ -32,10 +32,35 @@ def _positions(xbar, deltas):
     return None if xbar is None else (xbar[None] + deltas).contiguous()
 
 
+def _on_device(model, xbar_ref, xbar_alpha, deltas_ref, deltas_alpha):
+    """Whether the arrays are as XrayModel.kl_and_grad takes them (anything
+    else goes through array operations)."""
+    N = model.sky.N
+    if (xbar_alpha is not None) != model.sky.has_alpha or \
+            (deltas_alpha is not None) != model.sky.has_alpha:
+        return False
+    for x, d in ((xbar_ref, deltas_ref), (xbar_alpha, deltas_alpha)):
+        for t in (x, d):
+            if t is None:
+                continue
+            if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == model.dtype
+                    and t.get_device() == torch.cuda.current_device() and t.is_contiguous()
+                    and not (t.requires_grad and torch.is_grad_enabled())):
+                return False
+        if x is not None and (tuple(x.shape) != (N, N) or d.dim() != 3
+                              or tuple(d.shape[1:]) != (N, N)
+                              or d.shape[0] != deltas_ref.shape[0]):
+            return False
+    return True
+
+
 def kl_value_and_grad(model: XrayModel, xbar_ref, xbar_alpha, deltas_ref, deltas_alpha=None):
     """(KL value (float), (g_ref, g_alpha)) at the latent mean xbar for the
     sample offsets deltas (S, N, N); the S positions become the model's
     sample positions (for kl_solve)."""
+    if _on_device(model, xbar_ref, xbar_alpha, deltas_ref, deltas_alpha):
+        nll, squares, grads = model.kl_and_grad(xbar_ref, xbar_alpha, deltas_ref, deltas_alpha)
+        return float(np.mean(nll)) + 0.5 * squares / len(nll), grads
     pr = _positions(xbar_ref, deltas_ref)
     pa = _positions(xbar_alpha, deltas_alpha)
     nll, g_r, g_a = model.nll_and_grad_batch(pr, pa)

@@ -302,6 +302,29 @@ class XrayModel:
         return np.array(vals, dtype=np.float64), dev.like_input(g_ref, xi_ref), (
             dev.like_input(g_alpha, xi_ref) if g_alpha is not None else None)
 
+    def kl_and_grad(self, xbar_ref, xbar_alpha, deltas_ref, deltas_alpha):
+        """nll_and_grad_batch at the positions xbar + deltas with the sums of
+        the sampled KL on the device: (nll float64 numpy (S,), sum of all
+        squared positions, mean over the samples of gradient + position).
+        Contiguous device tensors of the model's dtype, xbar (N, N) and
+        deltas (S, N, N)."""
+        s = self.sky
+        S = self._batch_size(deltas_ref)
+        pos = [torch.empty_like(d) if d is not None else None for d in (deltas_ref, deltas_alpha)]
+        gs = [torch.empty_like(p) if p is not None else None for p in pos]
+        g_ref, g_alpha = self._grads()
+        nll = torch.empty(S, dtype=torch.float64, device="cuda")
+        _lib.call("jubik_model_kl_grad", self._model, S, dev.ptr(s.amp_ref), dev.ptr(s.amp_alpha),
+                  dev.ptr(xbar_ref), dev.ptr(xbar_alpha), dev.ptr(deltas_ref),
+                  dev.ptr(deltas_alpha), s.zm, s.mu, dev.ptr(s.dnu_dev), dev.ptr(nll),
+                  dev.ptr(pos[0]), dev.ptr(pos[1]), dev.ptr(gs[0]), dev.ptr(gs[1]),
+                  dev.ptr(g_ref), dev.ptr(g_alpha), dev.stream())
+        vals, prior = (ctypes.c_double * S)(), ctypes.c_double()
+        _lib.call("jubik_model_kl_result", self._model, vals, ctypes.byref(prior), dev.stream())
+        self._batch_S = S
+        self._batch_version = s.version
+        return np.array(vals, dtype=np.float64), prior.value, (g_ref, g_alpha)
+
     def metric_batch(self, v_ref, v_alpha=None):
         """S metric products J^T diag(1/lam) J v at the last gradient position;
         v of shape (S, N, N)."""
