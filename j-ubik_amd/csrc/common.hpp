@@ -180,6 +180,60 @@ __device__ __forceinline__ T gather_load(const Gather& g, int off) {
     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(g.r, off, 0, 0));
 }
 
+// Rows of a spectrum array seen by the lanes of a work-group: element (row,
+// column) at byte offset lane(row, column) + shift(rows), the first the
+// lane's own and the second uniform.  Rows before the first and at or past
+// the last read zero and are not stored: their offsets, taken modulo 2^32,
+// lie past the range that the hardware checks.  So a column's loads and
+// stores cost one addition each, or none with a constant shift of whole rows
+// inside the range (``step``), where bounds checks and 64-bit addresses
+// took six to eight instructions.  The column passes issue instructions for
+// half their time: at L = 384 the forward went from 2885 to 2053 vector
+// instructions a tile (with the tent weights read from LDS), the adjoint from
+// 2747 to 2023; measured forward / adjoint, 1024^2 x 4E 79 / 68 -> 79 / 63 us,
+// 1024^2 x 3E x 7 modules (L = 324) 523 / 480 -> 494 / 455 us, fold mode at
+// L = 432 53 / 45 -> 48 / 39 us.  Arrays stay below 1 GiB.
+template <typename T, int STRIDE>
+struct RowAccess {
+  typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  static constexpr int ROW = STRIDE * (int)sizeof(cplx<T>);  // bytes of a row
+  static constexpr int STREAM = 2;  // cache policy: non-temporal
+  __amdgpu_buffer_rsrc_t r;
+  __device__ RowAccess(const cplx<T>* p, int rows)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<cplx<T>*>(p), 0, (rows > 0 ? rows : 0) * ROW,
+                                            0x00020000)) {}
+  // Offset of the lane's element; columns outside the array (!ok) stay out
+  // of range whatever rows are added.
+  static __device__ __forceinline__ int lane(int row, int col, bool ok) {
+    return ok ? row * ROW + col * (int)sizeof(cplx<T>) : (int)0x80000000;
+  }
+  // The sum is kept whole in a register: a constant part split off into the
+  // instruction would be added without the wrap that rows before the first
+  // rely on.
+  static __device__ __forceinline__ int at(int lane_off, int rows) {
+    int off = lane_off + rows * ROW;
+    asm("" : "+v"(off));
+    return off;
+  }
+  template <int AUX = 0>
+  __device__ __forceinline__ cplx<T> load(int off, int step = 0) const {
+    if constexpr (sizeof(T) == 4)
+      return __builtin_bit_cast(cplx<T>,
+                                __builtin_amdgcn_raw_buffer_load_b64(r, off, step * ROW, AUX));
+    else
+      return __builtin_bit_cast(cplx<T>,
+                                __builtin_amdgcn_raw_buffer_load_b128(r, off, step * ROW, AUX));
+  }
+  template <int AUX = 0>
+  __device__ __forceinline__ void store(int off, cplx<T> v) const {
+    if constexpr (sizeof(T) == 4)
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, off, 0, AUX);
+    else
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, off, 0, AUX);
+  }
+};
+
 // Tile sizes: vectors per work-group so a tile of V vectors of length L at
 // the odd LDS stride occupies at most 52 KiB (16 float vectors at L = 384).
 #ifndef JUBIK_COL_TILE_BYTES

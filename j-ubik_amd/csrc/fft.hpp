@@ -531,6 +531,33 @@ struct Stage {
       }
     }
   }
+  // v[b][t] = src(b, lane, t * NB) and dst(b, lane, t * NB, value) with lane
+  // = at(vec, j) formed once per task.
+  template <class At, class Src>
+  static __device__ __forceinline__ void gather_rows(Regs& v, int tid, At at, Src src) {
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) {
+      int vec, j;
+      if (task(tid, b, vec, j)) {
+        const auto lane = at(vec, j);
+#pragma unroll
+        for (int t = 0; t < R; ++t) v[b][t] = src(lane, t * NB);
+      }
+    }
+  }
+  template <class At, class Dst>
+  static __device__ __forceinline__ void emit_rows(const Regs& v, int tid, At at, Dst dst) {
+    static_assert(Ns * R == L, "emit is for the last stage");
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) {
+      int vec, j;
+      if (task(tid, b, vec, j)) {
+        const auto lane = at(vec, j);
+#pragma unroll
+        for (int t = 0; t < R; ++t) dst(lane, t * NB, v[b][t]);
+      }
+    }
+  }
   // Last stage only (Ns * R == L): dst(vec, j + t * NB, value).
   template <class Dst>
   static __device__ __forceinline__ void emit(const Regs& v, int tid, Dst dst) {

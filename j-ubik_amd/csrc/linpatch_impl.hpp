@@ -45,8 +45,11 @@ __device__ __forceinline__ int cot_col(const LinGeom& g, int f) {
   if constexpr (!FOLD) {
     return f;
   } else {
-    int q = (f - g.mf + g.m) % g.Lw;
-    return q < 0 ? q + g.Lw : q;
+    // f - mf + m lies in [-Lw, 2 Lw) unless L > 3 Lw
+    int q = f - g.mf + g.m;
+    if (g.L > 3 * g.Lw) q %= g.Lw;
+    q += q < 0 ? g.Lw : 0;
+    return q >= g.Lw ? q - g.Lw : q;
   }
 }
 
@@ -334,6 +337,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
   __shared__ cplx<T> tw[L];
   __shared__ double red[NT / 64];
   __shared__ double total_s;
+  __shared__ T tent_s[MODE == COL_FWD ? L : 1];
   const int tid = threadIdx.x;
   constexpr int NTILE = (LH + V - 1) / V;
   const int nsmp = (MODE == COL_KERNEL) ? 1 : g.S;
@@ -396,57 +400,60 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
   // The kernel spectrum of this tile is loaded first: its latency then
   // overlaps the forward stages instead of stalling the multiply.
   typename FL::Regs kreg;
+  using Rows = RowAccess<T, L2P>;
+  auto in_range = [&](int vec) { return LH % V == 0 || k0 + vec < LH; };
   if constexpr (MODE != COL_KERNEL) {
-    const cplx<T>* ks = KT + spec * L2P * L;
-    FL::gather(kreg, tid, [&](int vec, int pos) -> cplx<T> {
-      const int k = k0 + vec;
-      return k < LH ? ks[pos * L2P + k] : cplx<T>{T(0), T(0)};
-    });
+    const Rows ks(KT + spec * L2P * L, L);
+    FL::gather_rows(
+        kreg, tid, [&](int vec, int j) { return Rows::lane(j, k0 + vec, in_range(vec)); },
+        [&](int lane, int rows) { return ks.load(lane, rows); });
   }
   // Image row of window row 0: the adjoint's input rows outside the image
   // are zero and were never stored; the forward's output rows there are
   // never read.
   const int row0 = start_x(g, p % g.n) - g.h - g.m;
-  const Gather gin = make_gather(in, MODE == COL_FWD ? (int64_t)g.H * L2P : 0);
-  const double tstep = tent_step(g.d);
-  auto load_col = [&](int vec, int pos) -> cplx<T> {
-    const int k = k0 + vec;
-    const cplx<T> zero = {T(0), T(0)};
-    if constexpr (MODE == COL_ADJ) {
-      if (k >= LH) return zero;
-      const int ir = row0 + cot_col<FOLD>(g, pos);
-      return (ir >= 0 && ir < g.H) ? ld_stream(&in[ir * L2P + k]) : zero;
-    } else if constexpr (MODE == COL_FWD) {
-      // the tent weight is applied after all loads are issued (tent_rows):
-      // a multiply here would make each task group wait for its loads
-      // before the next group's are issued
-      const int rr = pos - m;
-      const int ir = row0 + g.m + rr;
-      const bool ok = k < LH && rr >= 0 && rr < w && ir >= 0 && ir < g.H;
-      return gather_load<cplx<T>>(gin, gather_off<cplx<T>>(gin, ok, ir * L2P + k));
-    } else {
-      if (k >= LH) return zero;
-      const int rr = pos - m;
-      return (rr >= 0 && rr < w) ? ld_stream(&in[rr * L2P + k]) : zero;
-    }
-  };
-  // forward: window row pos - m carries its tent weight
-  auto tent_rows = [&](typename F0::Regs& regs) {
-    if constexpr (MODE == COL_FWD)
-      F0::for_each(regs, tid, [&](int, int pos, cplx<T>& val) {
-        val = cscale(val, tent_weight<T>(g.d, tstep, pos - m));
+  // Input rows: the forward's window rows inside the image, from frame
+  // position m on; the adjoint's image rows; the kernel's window rows.
+  const int top = MODE == COL_FWD ? row0 + g.m : 0;  // first window row
+  const int skip = top > 0 ? top : 0;
+  const Rows rin(in + (int64_t)skip * L2P,
+                 MODE == COL_FWD ? (top + w < g.H ? top + w : g.H) - skip
+                                 : MODE == COL_ADJ ? g.H : w);
+  const int shift = MODE == COL_FWD ? top - skip - m : MODE == COL_ADJ ? row0 : -m;
+  auto load_tile = [&](typename F0::Regs& regs) {
+    if constexpr (MODE == COL_ADJ && FOLD)
+      F0::gather(regs, tid, [&](int vec, int pos) {
+        return rin.load(Rows::at(Rows::lane(cot_col<FOLD>(g, pos), k0 + vec, in_range(vec)), row0));
       });
+    else
+      F0::gather_rows(
+          regs, tid, [&](int vec, int j) { return Rows::lane(j, k0 + vec, in_range(vec)); },
+          [&](int lane, int rows) { return rin.load(Rows::at(lane, rows + shift)); });
+  };
+  // Forward: window row pos - m carries its tent weight, read from LDS (and
+  // applied after all loads are issued: a multiply between them would make
+  // each task wait for its loads before the next one's are issued).
+  if constexpr (MODE == COL_FWD) {
+    const double tstep = tent_step(g.d);
+    for (int pos = tid; pos < L; pos += NT)
+      tent_s[pos] = pos >= m && pos < m + w ? tent_weight<T>(g.d, tstep, pos - m) : T(0);
+  }
+  auto tent_rows = [&](typename F0::Regs& regs) {
+    if constexpr (MODE == COL_FWD) {
+      __syncthreads();
+      F0::for_each(regs, tid, [&](int, int pos, cplx<T>& val) { val = cscale(val, tent_s[pos]); });
+    }
   };
   static_assert(F0::Ns == 1, "the first stage takes no twiddles");
   if constexpr (NS == 1) {
-    F0::gather(last, tid, load_col);
+    load_tile(last);
     store_twiddles();
     tent_rows(last);
     __syncthreads();
     F0::compute(last, tw, tid);
   } else {
     typename F0::Regs v0;
-    F0::gather(v0, tid, load_col);
+    load_tile(v0);
     store_twiddles();
     tent_rows(v0);
     F0::compute(v0, tw, tid);
@@ -508,19 +515,18 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
     using IL = Stage<T, L, true, NS - 1, V, VS, NT>;
     static_assert(I0::R == FL::R && I0::BPT == FL::BPT, "shared register layout");
     I0::compute(last, tw, tid);
-    cplx<T>* o = out + idx * L2P * (MODE == COL_ADJ ? w : lw);
-    auto store = [&](int vec, int pos, cplx<T> val) {
-      const int k = k0 + vec;
-      if (k >= LH) return;
-      if constexpr (MODE == COL_ADJ) {
-        const int r = pos - m;
-        if (r >= 0 && r < w) st_stream(&o[r * L2P + k], val);
-      } else {
-        // Output rows that fall outside the image are never read by the
-        // overlap pass (it gathers image rows only): not stored.
-        const int ir = row0 + pos;
-        if (ir >= 0 && ir < g.H) st_stream(&o[pos * L2P + k], val);
-      }
+    // Output rows: the adjoint's window rows; the forward's rows inside the
+    // image (the overlap pass gathers image rows only).
+    const int out0 = MODE == COL_FWD && row0 < 0 ? -row0 : 0;
+    const int outn = MODE == COL_ADJ ? w : (lw < g.H - row0 ? lw : g.H - row0) - out0;
+    const Rows ro(out + (idx * (MODE == COL_ADJ ? w : lw) + out0) * L2P, outn);
+    const int oshift = MODE == COL_ADJ ? -m : -out0;
+    auto store_tile = [&](auto stage, auto& vals) {
+      decltype(stage)::emit_rows(
+          vals, tid, [&](int vec, int j) { return Rows::lane(j, k0 + vec, in_range(vec)); },
+          [&](int lane, int rows, cplx<T> val) {
+            ro.template store<Rows::STREAM>(Rows::at(lane, rows + oshift), val);
+          });
     };
     // Fold mode, forward: the transformed columns go to LDS, one component
     // after the other, and output row q of the Lw window sums frame positions
@@ -557,16 +563,16 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
       for (int u = 0; u < FPT; ++u) {
         const int e = tid + u * NT;
         if (e >= V * lw) break;
-        const int k = k0 + (e & (V - 1)), q = e / V;
-        const int ir = row0 + q;
-        if (k < LH && ir >= 0 && ir < g.H) st_stream(&o[q * L2P + k], cplx<T>{re[u], im[u]});
+        const int vec = e & (V - 1), q = e / V;
+        ro.template store<Rows::STREAM>(
+            Rows::at(Rows::lane(q, k0 + vec, in_range(vec)), oshift), cplx<T>{re[u], im[u]});
       }
     };
     if constexpr (NS == 1) {
       if constexpr (kFoldOut)
         fold_out(I0{}, last);
       else
-        I0::emit(last, tid, store);
+        store_tile(I0{}, last);
     } else {
       typename IL::Regs v;
       __syncthreads();
@@ -578,7 +584,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
       if constexpr (kFoldOut)
         fold_out(IL{}, v);
       else
-        IL::emit(v, tid, store);
+        store_tile(IL{}, v);
     }
   }
   if constexpr (MODE == COL_ADJ) {
