@@ -72,6 +72,29 @@ __host__ __device__ constexpr int half_stride(int L) {
   return 16 * (q % 2 ? q : q + 1);
 }
 
+// Division of 32-bit unsigned integers by a number known before the launch:
+// floor(x m / 2^32) with m = floor(2^32 / d) is the quotient or one less.
+// Work-group indices are split by several such numbers before the first load
+// can be issued; the compiler's division is a chain of about 25 dependent
+// instructions each.
+struct Divisor {
+  uint32_t d, m;
+};
+__host__ __device__ __forceinline__ Divisor make_divisor(int d) {
+  return Divisor{(uint32_t)d, d > 1 ? (uint32_t)((1ull << 32) / (uint32_t)d) : 0xffffffffu};
+}
+__device__ __forceinline__ int div_by(const Divisor& v, int x) {
+  uint32_t q = __umulhi((uint32_t)x, v.m);
+  q += (uint32_t)x - q * v.d >= v.d ? 1 : 0;
+  return (int)q;
+}
+// x / d, and x % d left in x.
+__device__ __forceinline__ int div_mod(const Divisor& v, int& x) {
+  const int q = div_by(v, x);
+  x -= q * (int)v.d;
+  return q;
+}
+
 struct LinGeom {
   int H, W;       // sky grid
   int n;          // patches per axis
@@ -101,22 +124,34 @@ struct LinGeom {
   int S;          // samples per launch: jobs (s, mod, e) = s * J + mod * E + e
   int sky_shared; // adjoint into the GP: 1 = one sky (E, H, W) for every
                   // sample (metric at a base point), 0 = one sky per sample
+  Divisor by_n, by_d, by_P, by_E, by_J, by_S;  // set by the launchers
 };
+inline LinGeom with_divisors(LinGeom g) {
+  g.by_n = make_divisor(g.n);
+  g.by_d = make_divisor(g.d);
+  g.by_P = make_divisor(g.P);
+  g.by_E = make_divisor(g.E);
+  g.by_J = make_divisor(g.J);
+  g.by_S = make_divisor(g.S);
+  return g;
+}
 
 __device__ __forceinline__ int start_x(const LinGeom& g, int i) { return min(i * g.d, g.limx); }
 __device__ __forceinline__ int start_y(const LinGeom& g, int i) { return min(i * g.d, g.limy); }
-// Spectrum index of (job, patch): kernels are laid out (M, P, Ek); every
+// Spectrum index of (job of a sample, patch): kernels are laid out (M, P, Ek); every
 // sample of a batch shares them.
-__device__ __forceinline__ int64_t spec_index(const LinGeom& g, int job, int p) {
-  const int jm = job % g.J;
-  const int mod = jm / g.E, e = jm - mod * g.E;
+__device__ __forceinline__ int64_t spec_index(const LinGeom& g, int jm, int p) {
+  int e = jm;
+  const int mod = div_mod(g.by_E, e);
   return ((int64_t)mod * g.P + p) * g.Ek + (g.Ek == 1 ? 0 : e);
 }
 
 // Index of the shared row spectra of job z of sample smp: the job, or for a
 // forward signal shared by the modules the image (smp, energy).
 __device__ __forceinline__ int r1_image(const LinGeom& g, int smp, int z, bool fwd) {
-  return (fwd && g.x_shared) ? smp * g.E + z % g.E : smp * g.J + z;
+  int e = z;
+  if (fwd && g.x_shared) div_mod(g.by_E, e);
+  return (fwd && g.x_shared) ? smp * g.E + e : smp * g.J + z;
 }
 
 // Tent weight t of a 2d window (jubik/convolve.py:18-25): numpy

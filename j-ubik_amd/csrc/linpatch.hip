@@ -54,8 +54,9 @@ int linpatch_row_tile(int dtype, int L, int row_div) {
   return tile_vectors(JUBIK_ROW_TILE_BYTES, L, dtype == 0 ? 8 : 16) / row_div;
 }
 
-static int run(int dtype, const LinGeom& g, const LinBuffers& b, const LinCall& c,
+static int run(int dtype, const LinGeom& geom, const LinBuffers& b, const LinCall& c,
                hipStream_t s) {
+  const LinGeom g = with_divisors(geom);
   if (dtype != 0 && dtype != 1) return fail(kInvalidArgument, "dtype must be 0 (float32) or 1 (float64)");
   switch (g.L) {
 #define JUBIK_CASE(l) \

@@ -340,14 +340,17 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
   __shared__ T tent_s[MODE == COL_FWD ? L : 1];
   const int tid = threadIdx.x;
   constexpr int NTILE = (LH + V - 1) / V;
-  const int nsmp = (MODE == COL_KERNEL) ? 1 : g.S;
   int item = xcd_tile(blockIdx.x, gridDim.x);
-  const int smp = item % nsmp;
-  item /= nsmp;
-  const int k0 = (item % NTILE) * V;
-  item /= NTILE;
-  const int p = item % g.P;
-  const int z = item / g.P;
+  int smp = 0;
+  if constexpr (MODE != COL_KERNEL) {
+    smp = item;
+    item = div_mod(g.by_S, smp);
+  }
+  const int k0 = (int)((uint32_t)item % NTILE) * V;
+  int p = (int)((uint32_t)item / NTILE);
+  const int z = div_mod(g.by_P, p);
+  int pix = p;  // patch row
+  const int piy = div_mod(g.by_n, pix);
 
   int64_t idx, spec;
   if constexpr (MODE == COL_KERNEL) {
@@ -363,7 +366,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
   if constexpr (MODE == COL_KERNEL)
     in = R1 + idx * L2P * g.w;
   else
-    in = R1 + ((int64_t)r1_image(g, smp, z, MODE == COL_FWD) * g.n + p / g.n) * g.H * L2P;
+    in = R1 + ((int64_t)r1_image(g, smp, z, MODE == COL_FWD) * g.n + piy) * g.H * L2P;
   const int m = g.mf, w = g.w;
 
   // Twiddles are fetched into registers now and stored to LDS once the tile
@@ -397,21 +400,13 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
   using F0 = Stage<T, L, false, 0, V, VS, NT>;
   using FL = Stage<T, L, false, NS - 1, V, VS, NT>;
   typename FL::Regs last;
-  // The kernel spectrum of this tile is loaded first: its latency then
-  // overlaps the forward stages instead of stalling the multiply.
   typename FL::Regs kreg;
   using Rows = RowAccess<T, L2P>;
   auto in_range = [&](int vec) { return LH % V == 0 || k0 + vec < LH; };
-  if constexpr (MODE != COL_KERNEL) {
-    const Rows ks(KT + spec * L2P * L, L);
-    FL::gather_rows(
-        kreg, tid, [&](int vec, int j) { return Rows::lane(j, k0 + vec, in_range(vec)); },
-        [&](int lane, int rows) { return ks.load(lane, rows); });
-  }
   // Image row of window row 0: the adjoint's input rows outside the image
   // are zero and were never stored; the forward's output rows there are
   // never read.
-  const int row0 = start_x(g, p % g.n) - g.h - g.m;
+  const int row0 = start_x(g, pix) - g.h - g.m;
   // Input rows: the forward's window rows inside the image, from frame
   // position m on; the adjoint's image rows; the kernel's window rows.
   const int top = MODE == COL_FWD ? row0 + g.m : 0;  // first window row
@@ -444,9 +439,20 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
       F0::for_each(regs, tid, [&](int, int pos, cplx<T>& val) { val = cscale(val, tent_s[pos]); });
     }
   };
+  // The kernel spectrum of this tile: its loads are issued after the tile's
+  // own (loads complete in order) and overlap the forward stages.
+  auto load_spectrum = [&]() {
+    if constexpr (MODE != COL_KERNEL) {
+      const Rows ks(KT + spec * L2P * L, L);
+      FL::gather_rows(
+          kreg, tid, [&](int vec, int j) { return Rows::lane(j, k0 + vec, in_range(vec)); },
+          [&](int lane, int rows) { return ks.load(lane, rows); });
+    }
+  };
   static_assert(F0::Ns == 1, "the first stage takes no twiddles");
   if constexpr (NS == 1) {
     load_tile(last);
+    load_spectrum();
     store_twiddles();
     tent_rows(last);
     __syncthreads();
@@ -454,6 +460,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
   } else {
     typename F0::Regs v0;
     load_tile(v0);
+    load_spectrum();
     store_twiddles();
     tent_rows(v0);
     F0::compute(v0, tw, tid);
@@ -651,15 +658,13 @@ __device__ __forceinline__ int first_cover(int C, int len, int d, float rd) {
 // is contiguous.  Every argument is uniform over the work-group.
 __device__ __forceinline__ void cover_range(const LinGeom& g, int R, int len, int& lo,
                                             int& count) {
-  lo = g.n;
-  count = 0;
-  for (int ix = 0; ix < g.n; ++ix) {
-    const int s = start_x(g, ix);
-    if (R >= s && R < s + len) {
-      lo = min(lo, ix);
-      ++count;
-    }
-  }
+  // Unclamped starts ix d <= R < ix d + len; only the last start is clamped.
+  const int last = g.n - 1;
+  lo = R < len ? 0 : div_by(g.by_d, R - len) + 1;
+  int hi = min(div_by(g.by_d, R), last);
+  if (R >= g.limx) hi = last;
+  if (lo >= last) lo = R < start_x(g, last) + len ? last : g.n;
+  count = max(hi - lo + 1, 0);
 }
 
 // buf[v][k] for v < V, k < L: the sum over the covering patch rows ci of
@@ -792,7 +797,9 @@ __global__ __launch_bounds__(NTO) void lp_fwd_out(LinGeom g, const cplx<T>* __re
 #pragma unroll
   for (int t = 0; t < JPT; ++t) acc[t] = T(0);
   const int64_t row = ((int64_t)job * g.H + i) * g.W;
-  const int64_t rowd = ((int64_t)(job % g.J) * g.H + i) * g.W;
+  int jm = job;  // job of its sample
+  div_mod(g.by_J, jm);
+  const int64_t rowd = ((int64_t)jm * g.H + i) * g.W;
   // metric: the base-point lam of (mod, e), or of this job's own sample
   // when the samples have their own base points (sky_shared = 0)
   const int64_t rowl = g.sky_shared ? rowd : row;
@@ -966,7 +973,8 @@ __global__ __launch_bounds__(NTO) void lp_adj_out(LinGeom g, const cplx<T>* __re
   // EPI 0 with a shared input and EPI 1: the jobs (s, mod, e) of image
   // blockIdx.y = s * E + e, summed over modules; EPI 0 otherwise: job
   // blockIdx.y.
-  const int smp = blockIdx.y / g.E, eb = blockIdx.y - smp * g.E;
+  int eb = blockIdx.y;
+  const int smp = div_mod(g.by_E, eb);
   int jb = smp * g.J + eb, je = (smp + 1) * g.J, jstep = g.E;
   if (EPI == 0 && !g.x_shared) {
     jb = blockIdx.y;
@@ -1033,7 +1041,8 @@ __global__ __launch_bounds__(NTO) void lp_adj_out(LinGeom g, const cplx<T>* __re
     const cplx<T>* base = R2 + (int64_t)job * g.P * g.w * L2P;
     T dn = T(0);
     if constexpr (EPI == 3) {
-      const int e = (job - jb) % g.E;
+      int e = job - jb;
+      div_mod(g.by_E, e);
       const int simg = g.sky_shared ? e : blockIdx.y * g.E + e;
       const T* srow = sky + ((int64_t)simg * g.H + i) * g.W;
 #pragma unroll

@@ -249,18 +249,19 @@ __global__ __launch_bounds__(MNT) void lp_cols_mfma(LinGeom g, const bf16x8* __r
   };
   auto locate = [&](int item) {
     Item it;
-    const int smp = item % g.S;
-    item /= g.S;
+    int smp = item;
+    item = div_mod(g.by_S, smp);
     it.k0 = (item % MNTILE) * MV;
-    item /= MNTILE;
-    const int p = item % g.P;
-    const int z = item / g.P;
+    int p = item / MNTILE;
+    const int z = div_mod(g.by_P, p);
+    int pix = p;
+    const int piy = div_mod(g.by_n, pix);
     it.idx = (int64_t)(smp * g.J + z) * g.P + p;
-    it.rows = ((int64_t)r1_image(g, smp, z, !ADJ) * g.n + p / g.n) * g.H;
+    it.rows = ((int64_t)r1_image(g, smp, z, !ADJ) * g.n + piy) * g.H;
     it.spec = spec_index(g, z, p);
     // image row of frame row 0: rows outside the image are zero on input
     // (never stored) and never read on output
-    it.row0 = start_x(g, p % g.n) - g.h - g.m;
+    it.row0 = start_x(g, pix) - g.h - g.m;
     return it;
   };
   // element e = tid + u * MNT of a tile: column e % MV, frame row e / MV
