@@ -215,6 +215,16 @@ __device__ __forceinline__ T gather_load(const Gather& g, int off) {
     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(g.r, off, 0, 0));
 }
 
+template <typename T, int AUX = 0>
+__device__ __forceinline__ cplx<T> buffer_load(__amdgpu_buffer_rsrc_t r, int off, int uniform = 0) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b64(r, off, uniform, AUX));
+  else
+    return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b128(r, off, uniform, AUX));
+}
+constexpr int kStream = 2;                     // cache policy: non-temporal
+constexpr int kOutOfRange = (int)0x80000000;  // lies past every range
+
 // Rows of a spectrum array seen by the lanes of a work-group: element (row,
 // column) at byte offset lane(row, column) + shift(rows), the first the
 // lane's own and the second uniform.  Rows before the first and at or past
@@ -233,7 +243,6 @@ struct RowAccess {
   typedef unsigned int u2 __attribute__((ext_vector_type(2)));
   typedef unsigned int u4 __attribute__((ext_vector_type(4)));
   static constexpr int ROW = STRIDE * (int)sizeof(cplx<T>);  // bytes of a row
-  static constexpr int STREAM = 2;  // cache policy: non-temporal
   __amdgpu_buffer_rsrc_t r;
   __device__ RowAccess(const cplx<T>* p, int rows)
       : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<cplx<T>*>(p), 0, (rows > 0 ? rows : 0) * ROW,
@@ -241,7 +250,7 @@ struct RowAccess {
   // Offset of the lane's element; columns outside the array (!ok) stay out
   // of range whatever rows are added.
   static __device__ __forceinline__ int lane(int row, int col, bool ok) {
-    return ok ? row * ROW + col * (int)sizeof(cplx<T>) : (int)0x80000000;
+    return ok ? row * ROW + col * (int)sizeof(cplx<T>) : kOutOfRange;
   }
   // The sum is kept whole in a register: a constant part split off into the
   // instruction would be added without the wrap that rows before the first
@@ -253,12 +262,7 @@ struct RowAccess {
   }
   template <int AUX = 0>
   __device__ __forceinline__ cplx<T> load(int off, int step = 0) const {
-    if constexpr (sizeof(T) == 4)
-      return __builtin_bit_cast(cplx<T>,
-                                __builtin_amdgcn_raw_buffer_load_b64(r, off, step * ROW, AUX));
-    else
-      return __builtin_bit_cast(cplx<T>,
-                                __builtin_amdgcn_raw_buffer_load_b128(r, off, step * ROW, AUX));
+    return buffer_load<T, AUX>(r, off, step * ROW);
   }
   template <int AUX = 0>
   __device__ __forceinline__ void store(int off, cplx<T> v) const {

@@ -532,7 +532,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
       decltype(stage)::emit_rows(
           vals, tid, [&](int vec, int j) { return Rows::lane(j, k0 + vec, in_range(vec)); },
           [&](int lane, int rows, cplx<T> val) {
-            ro.template store<Rows::STREAM>(Rows::at(lane, rows + oshift), val);
+            ro.template store<kStream>(Rows::at(lane, rows + oshift), val);
           });
     };
     // Fold mode, forward: the transformed columns go to LDS, one component
@@ -571,7 +571,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
         const int e = tid + u * NT;
         if (e >= V * lw) break;
         const int vec = e & (V - 1), q = e / V;
-        ro.template store<Rows::STREAM>(
+        ro.template store<kStream>(
             Rows::at(Rows::lane(q, k0 + vec, in_range(vec)), oshift), cplx<T>{re[u], im[u]});
       }
     };
@@ -667,14 +667,66 @@ __device__ __forceinline__ void cover_range(const LinGeom& g, int R, int len, in
   count = max(hi - lo + 1, 0);
 }
 
+// acc[t] += the sum over the patch columns iy that cover canvas column C + t
+// NTO (ascending), of the pairs [q0, q0 + V) held in ``buf``: real parts of
+// even, imaginary parts of odd columns, at window column c = C - start_y(iy)
+// < len.  value(col, c) reads window column c of a transformed vector's
+// component.  Steps are uniform (ceil(len / d) columns at most, one more when
+// the last start is clamped) and outermost, so the LDS reads of a thread's
+// columns overlap; columns that do not cover read an element in range and add
+// zero.
+template <typename T, int V, int VS, int N, int JPT, class Value>
+__device__ __forceinline__ void sum_first_columns(T (&acc)[JPT], const T* buf, const LinGeom& g,
+                                                  int len, int C, int q0, int steps, float rd,
+                                                  Value value) {
+  const int last = g.n - 1;
+  const int ahead = max(last * g.d - g.limy, 0);  // the last start lies this much earlier
+  int iy[N], c[N];
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    iy[t] = first_cover(C + t * NTO, len, g.d, rd);
+    c[t] = C + t * NTO - iy[t] * g.d;
+  }
+#pragma unroll 1
+  for (int k = 0; k < steps; ++k) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      const int cc = c[t] + (iy[t] == last ? ahead : 0);
+      const int v = (iy[t] >> 1) - q0;
+      const bool ok = iy[t] <= last && (unsigned)cc < (unsigned)len && (unsigned)v < (unsigned)V;
+      const T x = value(buf + (ok ? 2 * v * VS + (iy[t] & 1) : 0), ok ? cc : 0);
+      acc[t] += ok ? x : T(0);
+      ++iy[t];
+      c[t] -= g.d;
+    }
+  }
+}
+// The first N of a thread's columns lie inside the image: grids of at most one
+// or two times NTO columns skip the others (256^2, a metric of 32 tangents:
+// 185 us with all four columns of a thread, 176 us with one).
+template <typename T, int V, int VS, int JPT, class Value>
+__device__ __forceinline__ void sum_columns(T (&acc)[JPT], const T* buf, const LinGeom& g, int len,
+                                            int C, int q0, int steps, float rd, Value value) {
+  if (g.W <= NTO)
+    sum_first_columns<T, V, VS, 1>(acc, buf, g, len, C, q0, steps, rd, value);
+  else if (g.W <= 2 * NTO)
+    sum_first_columns<T, V, VS, 2>(acc, buf, g, len, C, q0, steps, rd, value);
+  else
+    sum_first_columns<T, V, VS, JPT>(acc, buf, g, len, C, q0, steps, rd, value);
+}
+__device__ __forceinline__ int cover_steps(const LinGeom& g, int len) {
+  return div_by(g.by_d, len + g.d - 1) + ((g.n - 1) * g.d > g.limy ? 1 : 0);
+}
+
 // buf[v][k] for v < V, k < L: the sum over the covering patch rows ci of
 // wt_ci * (A_ci(k) + i B_ci(k)), where A and B are the full spectra of patch
 // columns iy = 2(q0 + v) and 2(q0 + v) + 1 rebuilt from their half spectra
 // (X(L - kk) = conj X(kk); slot 0 holds the real pair (X[0], X[L/2])).
 // Patch (ix, iy) row f starts at base + ((iy n + ix) nrows + f) L2p.  Each
 // half-spectrum element is loaded once and fills k = kk and k = L - kk; the
-// loads of up to three covering rows are in flight together.  Weights are tent[f] when WEIGHTED.
-// Patch offsets (2q + 1) n nrows L2p stay below 2^31 for n <= 64, L <= 384.
+// loads of up to CH covering rows are in flight together, through one buffer
+// resource per row: no bounds test and no address arithmetic per load.
+// Weights are tent[f] when WEIGHTED.
 template <typename T, int L, bool WEIGHTED>
 __device__ __forceinline__ void sum_pair_spectra(cplx<T>* buf, const cplx<T>* __restrict__ base,
                                                  const LinGeom& g, int nrows, int R, int lo,
@@ -684,24 +736,30 @@ __device__ __forceinline__ void sum_pair_spectra(cplx<T>* buf, const cplx<T>* __
   constexpr int V = OT::V, LH = OT::LH, GPT = OT::GPT;
   constexpr int VS = lds_stride(L, V);
   constexpr int L2P = half_stride(L);
-  // Covering rows per load batch: the forward's windows of L <= 3d rows meet
-  // a canvas row at most 3 times in the common geometries, and all three are
-  // loaded together.  The adjoint's windows of w = 2d rows meet it twice;
-  // they are loaded one after the other, which keeps the chained epilogue
-  // at 4 waves per SIMD instead of 3 (measured at 1024^2 x 4E, L = 384:
-  // 44 -> 38 us).
-  constexpr int CH = WEIGHTED ? 1 : 3;
-  const int npair = (g.n + 1) / 2;
-  const int pstride = nrows * L2P;  // n <= 64, L <= 384: offsets fit in 31 bits
+  // Covering rows per load batch.  The forward's rows come one after the
+  // other: of three or four at once each takes GPT pairs of registers, and the
+  // waves those cost hide more latency than the loads in flight (1, 2, 3, 4 at
+  // once: 1024^2 x 3E x 7 modules, L = 324, 306, 340, 333, 342 us; 2048^2 x 4E
+  // x 4 samples, L = 384, 626, 710, 677, 708 us).  The adjoint's windows of w
+  // = 2d rows meet a row twice, and both are loaded together (1, 2 at once:
+  // 218, 211 and 481, 453 us).  Before, with an address and a branch per load
+  // and a divergent loop per output column, 344 and 785 us forward, 249 and
+  // 588 us adjoint.
+  constexpr int CH = WEIGHTED ? 2 : 1;
+  // Patch columns of this batch and the bytes between two of them (below 2
+  // GiB for the 2 V columns); rows that do not cover have an empty range.
+  const int ncol = min(2 * V, g.n - 2 * q0);
+  const int pcol = g.n * nrows * L2P * (int)sizeof(cplx<T>);
+  base += (int64_t)(2 * q0) * g.n * nrows * L2P;
   int oa[GPT], ob[GPT];
 #pragma unroll
   for (int u = 0; u < GPT; ++u) {
     const int e = tid + u * NTO;
     const int v = e / LH, kk = e - (e / LH) * LH;
-    const int q = q0 + v;
-    const bool ok = (V * LH % NTO == 0 || e < V * LH) && q < npair;
-    oa[u] = ok ? 2 * q * g.n * pstride + kk : -1;
-    ob[u] = ok && 2 * q + 1 < g.n ? (2 * q + 1) * g.n * pstride + kk : -1;
+    const bool ok = V * LH % NTO == 0 || e < V * LH;
+    const int o = 2 * v * pcol + kk * (int)sizeof(cplx<T>);
+    oa[u] = ok && 2 * v < ncol ? o : kOutOfRange;
+    ob[u] = ok && 2 * v + 1 < ncol ? o + pcol : kOutOfRange;
   }
   cplx<T> A[GPT], B[GPT];
 #pragma unroll
@@ -711,19 +769,18 @@ __device__ __forceinline__ void sum_pair_spectra(cplx<T>* buf, const cplx<T>* __
     T wt[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      wt[c] = T(0);
+      const bool in = c0 + c < nc;
+      const int ix = in ? lo + c0 + c : lo;
+      const int f = R - start_x(g, ix);
+      wt[c] = WEIGHTED ? tent[f] : T(1);
+      const int row = (ix * nrows + f) * L2P;
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<cplx<T>*>(base + row), 0,
+          in ? ncol * pcol - row * (int)sizeof(cplx<T>) : 0, 0x00020000);
 #pragma unroll
-      for (int u = 0; u < GPT; ++u) a[c][u] = b[c][u] = cplx<T>{T(0), T(0)};
-      if (c0 + c < nc) {
-        const int ix = lo + c0 + c;
-        const int f = R - start_x(g, ix);
-        wt[c] = WEIGHTED ? tent[f] : T(1);
-        const cplx<T>* rowp = base + ((int64_t)ix * nrows + f) * L2P;
-#pragma unroll
-        for (int u = 0; u < GPT; ++u) {
-          if (oa[u] >= 0) a[c][u] = ld_stream(&rowp[oa[u]]);
-          if (ob[u] >= 0) b[c][u] = ld_stream(&rowp[ob[u]]);
-        }
+      for (int u = 0; u < GPT; ++u) {
+        a[c][u] = buffer_load<T, kStream>(r, oa[u]);
+        b[c][u] = buffer_load<T, kStream>(r, ob[u]);
       }
     }
 #pragma unroll
@@ -804,6 +861,7 @@ __global__ __launch_bounds__(NTO) void lp_fwd_out(LinGeom g, const cplx<T>* __re
   // when the samples have their own base points (sky_shared = 0)
   const int64_t rowl = g.sky_shared ? rowd : row;
   const float rd = 1.0f / (float)g.d;
+  const int steps = cover_steps(g, lw);
   T ex_v[JPT], lam_v[JPT];
   int cnt_v[JPT];
   const int npair = (g.n + 1) / 2;
@@ -839,33 +897,18 @@ __global__ __launch_bounds__(NTO) void lp_fwd_out(LinGeom g, const cplx<T>* __re
     }
     __syncthreads();
     fft_lds<T, L, V, VS, NTO, true, kFewVectorPlan<L, V, NTO>>(buf, tw, tid);
-#pragma unroll
-    for (int t = 0; t < JPT; ++t) {
-      const int j = tid + t * NTO;
-      if (j < g.W) {
-        const int C = j + g.h + g.m;
-        T s = T(0);
-        for (int iy = first_cover(C, lw, g.d, rd); iy < g.n; ++iy) {
-          const int sy = start_y(g, iy);
-          if (sy > C) break;
-          const int c = C - sy;
-          const int v = (iy >> 1) - q0;
-          if (c < lw && v >= 0 && v < V) {
-            if constexpr (FOLD) {
-              const int cf = c - g.m + g.mf;
-              cplx<T> z = buf[v * VS + cf];
-              if (cf + lw < L) z = cadd(z, buf[v * VS + cf + lw]);
-              if (cf >= lw) z = cadd(z, buf[v * VS + cf - lw]);
-              s += (iy & 1) ? z.im : z.re;
-            } else {
-              const cplx<T> z = buf[v * VS + c];
-              s += (iy & 1) ? z.im : z.re;
-            }
-          }
-        }
-        acc[t] += s;
-      }
-    }
+    sum_columns<T, V, VS>(acc, reinterpret_cast<const T*>(buf), g, lw, tid + g.h + g.m, q0, steps,
+                          rd, [&](const T* col, int c) {
+                            if constexpr (FOLD) {
+                              const int cf = c - g.m + g.mf;
+                              T z = col[2 * cf];
+                              if (cf + lw < L) z += col[2 * (cf + lw)];
+                              if (cf >= lw) z += col[2 * (cf - lw)];
+                              return z;
+                            } else {
+                              return col[2 * c];
+                            }
+                          });
     __syncthreads();
   };
   pass(0, std::true_type{});
@@ -993,6 +1036,7 @@ __global__ __launch_bounds__(NTO) void lp_adj_out(LinGeom g, const cplx<T>* __re
   // loads.
   T sky_v[JPT];
   const float rd = 1.0f / (float)g.d;
+  const int steps = cover_steps(g, g.w);
   // One batch of V patch-column pairs of one job; the first batch of the
   // first job is peeled into straight-line code (see lp_fwd_out).
   auto pass = [&](const cplx<T>* base, int q0, auto first) {
@@ -1016,25 +1060,9 @@ __global__ __launch_bounds__(NTO) void lp_adj_out(LinGeom g, const cplx<T>* __re
     }
     __syncthreads();
     fft_lds<T, L, V, VS, NTO, true, kFewVectorPlan<L, V, NTO>>(buf, tw, tid);
-#pragma unroll
-    for (int t = 0; t < JPT; ++t) {
-      const int j = tid + t * NTO;
-      if (j < g.W) {
-        const int Cp = j + g.h;
-        T s = T(0);
-        for (int iy = first_cover(Cp, g.w, g.d, rd); iy < g.n; ++iy) {
-          const int sy = start_y(g, iy);
-          if (sy > Cp) break;
-          const int c = Cp - sy;
-          const int v = (iy >> 1) - q0;
-          if (c < g.w && v >= 0 && v < V) {
-            const cplx<T> z = buf[v * VS + g.mf + c];
-            s += tent_s[c] * ((iy & 1) ? z.im : z.re);
-          }
-        }
-        tmp[t] += s;
-      }
-    }
+    sum_columns<T, V, VS>(tmp, reinterpret_cast<const T*>(buf) + 2 * g.mf, g, g.w, tid + g.h, q0,
+                          steps, rd,
+                          [&](const T* col, int c) { return tent_s[c] * col[2 * c]; });
     __syncthreads();
   };
   for (int job = jb; job < je; job += jstep) {
