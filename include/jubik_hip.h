@@ -154,6 +154,19 @@ int jubik_readout_gather(int dtype, const void* x, const int64_t* index, int64_t
                          void* stream);
 int jubik_readout_scatter(int dtype, const void* v, const int64_t* index, int64_t nnz, int64_t n,
                           void* out, void* stream);
+/* The same for several modules in one launch, by bit words: bit b of
+ * words[i * nwords + k], nwords = ceil(pixels / 64), says whether pixel 64 k +
+ * b of module i is kept (bits from ``pixels`` on are zero), and
+ * before[i * nwords + k] counts the kept pixels of module i before that word
+ * (device arrays).  Module i of x starts at x + i * stride elements, stride >=
+ * pixels; out[i] and v[i] (host arrays of device pointers) hold its kept
+ * pixels. */
+int jubik_readout_gather_words(int dtype, int64_t modules, const uint64_t* words,
+                               const int64_t* before, int64_t pixels, const void* x,
+                               int64_t stride, void* const* out, void* stream);
+int jubik_readout_scatter_words(int dtype, int64_t modules, const uint64_t* words,
+                                const int64_t* before, int64_t pixels, const void* const* v,
+                                void* out, void* stream);
 /* Mock counts: counts[i] ~ Poisson(lam[i]) for n device values, as the
  * mock-data generator draws them per read-out key
  * (jubik/data.py:139-145, jax.random.poisson).  A draw is a pure function of
@@ -168,6 +181,13 @@ int jubik_poisson_sample(int dtype, const void* lam, int64_t n, uint64_t seed, i
  * NULL).  ``work``: JUBIK_POISSON_WORK_BYTES of device memory. */
 int jubik_poisson_nll_grad(int dtype, const void* lam, const void* data, int64_t n, double* nll,
                            void* grad, void* work, void* stream);
+/* jubik_poisson_nll_grad of nseg arrays (the read-out keys), sizes n[i], in
+ * one launch: nll[i] (device doubles) is what the call for that array alone
+ * gives.  lam, data, n and grad (NULL, or pointers that may be NULL) are host
+ * arrays; ``work``: nseg * JUBIK_POISSON_WORK_BYTES of device memory. */
+int jubik_poisson_nll_grad_segments(int dtype, int64_t nseg, const void* const* lam,
+                                    const void* const* data, const int64_t* n, double* nll,
+                                    void* const* grad, void* work, void* stream);
 /* jubik_poisson_nll_grad without a workspace argument and without any
  * allocation: no counterpart in the reference; for callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops,

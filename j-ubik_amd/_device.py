@@ -89,5 +89,10 @@ def ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
 
 
+def ptrs(tensors):
+    """Host array of the tensors' device pointers."""
+    return (C.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
 def stream():
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)

@@ -40,6 +40,10 @@ SIGNATURES = {
     "jubik_exposure_apply": [_int, _vp, _i64, _vp, _i64, _vp, _i64, _vp],
     "jubik_readout_gather": [_int, _vp, _vp, _i64, _vp, _vp],
     "jubik_readout_scatter": [_int, _vp, _vp, _i64, _i64, _vp, _vp],
+    "jubik_readout_gather_words": [_int, _i64, _vp, _vp, _i64, _vp, _i64, C.POINTER(_vp), _vp],
+    "jubik_readout_scatter_words": [_int, _i64, _vp, _vp, _i64, C.POINTER(_vp), _vp, _vp],
+    "jubik_poisson_nll_grad_segments": [_int, _i64, C.POINTER(_vp), C.POINTER(_vp),
+                                        C.POINTER(_i64), _vp, C.POINTER(_vp), _vp, _vp],
     "jubik_poisson_nll_grad": [_int, _vp, _vp, _i64, _vp, _vp, _vp, _vp],
     "jubik_poisson_metric": [_int, _vp, _vp, _i64, _int, _vp, _vp],
     "jubik_poisson_nll_grad_noalloc": [_int, _vp, _vp, _i64, _vp, _vp, _vp],

@@ -723,6 +723,48 @@ int jubik_readout_scatter(int dtype, const void* v, const int64_t* index, int64_
   return readout_scatter(dtype, v, index, nnz, n, out, as_stream(stream));
 }
 
+static int readout_words_call(int dtype, bool gather, int64_t modules, const uint64_t* words,
+                              const int64_t* before, int64_t pixels, const void* x,
+                              int64_t stride, const void* const* v, void* stream) {
+  if (dtype != 0 && dtype != 1) return fail(kInvalidArgument, "dtype must be 0 or 1");
+  if (modules < 0 || pixels < 0 || stride < pixels) return fail(kInvalidArgument, "invalid sizes");
+  // the transpose writes the pixels that the words describe and no others
+  if (!gather && stride != pixels) return fail(kInvalidArgument, "invalid sizes");
+  if (modules && pixels && (!words || !before || !x || !v))
+    return fail(kInvalidArgument, "NULL argument");
+  if (pixels > (int64_t)1 << 36) return fail(kUnsupported, "module too large");
+  return readout_words(dtype, gather, modules, words, before, (pixels + 63) / 64,
+                       const_cast<void*>(x), stride, const_cast<void* const*>(v),
+                       as_stream(stream));
+}
+
+int jubik_readout_gather_words(int dtype, int64_t modules, const uint64_t* words,
+                               const int64_t* before, int64_t pixels, const void* x,
+                               int64_t stride, void* const* out, void* stream) {
+  return readout_words_call(dtype, true, modules, words, before, pixels, x, stride, out, stream);
+}
+
+int jubik_readout_scatter_words(int dtype, int64_t modules, const uint64_t* words,
+                                const int64_t* before, int64_t pixels, const void* const* v,
+                                void* out, void* stream) {
+  return readout_words_call(dtype, false, modules, words, before, pixels, out, pixels, v, stream);
+}
+
+int jubik_poisson_nll_grad_segments(int dtype, int64_t nseg, const void* const* lam,
+                                    const void* const* data, const int64_t* n, double* nll,
+                                    void* const* grad, void* work, void* stream) {
+  if (dtype != 0 && dtype != 1) return fail(kInvalidArgument, "dtype must be 0 or 1");
+  if (nseg < 0) return fail(kInvalidArgument, "negative size");
+  if (nseg && (!lam || !data || !n || !nll || !work))
+    return fail(kInvalidArgument, "NULL argument");
+  for (int64_t i = 0; i < nseg; ++i) {
+    if (n[i] < 0) return fail(kInvalidArgument, "negative size");
+    if (n[i] && (!lam[i] || !data[i])) return fail(kInvalidArgument, "NULL argument");
+  }
+  return poisson_nll_grad_segments(dtype, nseg, lam, data, n, nll, grad, (double*)work,
+                                   as_stream(stream));
+}
+
 int jubik_poisson_sample(int dtype, const void* lam, int64_t n, uint64_t seed, int32_t* counts,
                          void* stream) {
   if (dtype != 0 && dtype != 1) return fail(kInvalidArgument, "dtype must be 0 or 1");

@@ -46,23 +46,114 @@ __global__ __launch_bounds__(RNT) void k_scatter(const T* __restrict__ v,
     out[idx[k]] = v[k];
 }
 
-// partial[b] = sum over this block's elements of (lam - d log lam);
-// grad = 1 - d / lam.
+// Read-out of all modules in one launch.  The kept pixels of a module are a
+// bit per pixel, 64 to a word, with the number of kept pixels before each
+// word: a wave takes a word, and a lane's place among the kept pixels is the
+// count of the bits below its own.  That is 16 bytes of index per 64 pixels
+// where a list of kept positions takes 512, reads and writes both run in
+// order, and the transpose writes every pixel once instead of filling first.
+// kWords words per wave are in flight together.  Bound by its traffic; 512^2 x
+// 3E x 7 modules in FP64, gather + transpose, with a launch per module and the
+// list of positions 38 + 59 us, so 15 + 15 us (6 TB/s).
+constexpr int kReadoutSegs = 16;  // modules per launch
+constexpr int kWords = 8;
+template <typename P>
+struct ModulePtrs {
+  P v[kReadoutSegs];
+};
+
+// grid (ceil(nwords / (kWords RNT / 64)), modules).  GATHER: v[i][rank] =
+// x[i stride + p] for kept p; else x[i stride + p] = kept ? v[i][rank] : 0, p <
+// stride.
+template <typename T, bool GATHER, typename V = std::conditional_t<GATHER, T, const T>,
+          typename X = std::conditional_t<GATHER, const T, T>>
+__global__ __launch_bounds__(RNT) void k_readout_words(const uint64_t* __restrict__ words,
+                                                       const int64_t* __restrict__ before,
+                                                       int64_t nwords, X* __restrict__ x,
+                                                       int64_t stride, ModulePtrs<V*> v) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t w0 = ((int64_t)blockIdx.x * (RNT / 64) + wave) * kWords;
+  words += blockIdx.y * nwords;
+  before += blockIdx.y * nwords;
+  x += blockIdx.y * stride;
+  V* vm = v.v[blockIdx.y];
+  T val[kWords];
+  int64_t at[kWords];
+  bool on[kWords];
+#pragma unroll
+  for (int i = 0; i < kWords; ++i) {
+    const int64_t w = w0 + i < nwords ? w0 + i : 0;
+    const uint64_t bits = w0 + i < nwords ? words[w] : 0;
+    on[i] = (bits >> lane) & 1;
+    at[i] = before[w] + __popcll(bits & ((1ull << lane) - 1));
+  }
+#pragma unroll
+  for (int i = 0; i < kWords; ++i)
+    val[i] = on[i] ? (GATHER ? x[(w0 + i) * 64 + lane] : vm[at[i]]) : T(0);
+#pragma unroll
+  for (int i = 0; i < kWords; ++i) {
+    const int64_t p = (w0 + i) * 64 + lane;
+    if constexpr (GATHER) {
+      if (on[i]) vm[at[i]] = val[i];
+    } else {
+      if (p < stride) x[p] = val[i];
+    }
+  }
+}
+
+// Sum of (lam - d log lam) over the elements of block b of ``blocks``; grad =
+// 1 - d / lam.
+template <typename T>
+__device__ __forceinline__ double poisson_block(const T* __restrict__ lam,
+                                                const T* __restrict__ d, int64_t n,
+                                                T* __restrict__ grad, int blocks) {
+  double acc = 0.0;
+  for (int64_t k = blockIdx.x * (int64_t)RNT + threadIdx.x; k < n; k += (int64_t)blocks * RNT) {
+    const T l = lam[k], dk = d[k];
+    acc += (double)l - (double)dk * log((double)l);
+    if (grad) grad[k] = T(1) - dk / l;
+  }
+  return acc;
+}
+
+// partial[b] = the sum of block b.
 template <typename T>
 __global__ __launch_bounds__(RNT) void k_poisson(const T* __restrict__ lam,
                                                  const T* __restrict__ d, int64_t n,
                                                  T* __restrict__ grad,
                                                  double* __restrict__ partial) {
   __shared__ double red[RNT / 64];
-  double acc = 0.0;
-  for (int64_t k = blockIdx.x * (int64_t)RNT + threadIdx.x; k < n;
-       k += (int64_t)gridDim.x * RNT) {
-    const T l = lam[k], dk = d[k];
-    acc += (double)l - (double)dk * log((double)l);
-    if (grad) grad[k] = T(1) - dk / l;
-  }
-  acc = block_sum<RNT>(acc, red);
+  const double acc = block_sum<RNT>(poisson_block(lam, d, n, grad, gridDim.x), red);
   if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+}
+
+// Blocks of the Poisson reduction for n elements: one partial per block.
+__host__ __device__ __forceinline__ int poisson_blocks(int64_t n) {
+  const int64_t b = (n + RNT - 1) / RNT;
+  return (int)(b < 1 ? 1 : b > RBLOCKS ? RBLOCKS : b);
+}
+
+// Several arrays (the read-out keys) in one launch, grid (most blocks, arrays):
+// each is reduced by the blocks, and in the order, that it has alone.  512^2 x
+// 3E x 7 modules in FP64: seven launches of the two kernels 74 us, one of each
+// 36 us, and the call waits for the device once instead of seven times.
+template <typename T>
+struct PoissonSegs {
+  const T* lam[kReadoutSegs];
+  const T* d[kReadoutSegs];
+  T* grad[kReadoutSegs];
+  int64_t n[kReadoutSegs];
+};
+template <typename T>
+__global__ __launch_bounds__(RNT) void k_poisson_segments(PoissonSegs<T> t,
+                                                          double* __restrict__ partial) {
+  __shared__ double red[RNT / 64];
+  const int i = blockIdx.y;
+  const int blocks = poisson_blocks(t.n[i]);
+  if ((int)blockIdx.x >= blocks) return;
+  const double acc =
+      block_sum<RNT>(poisson_block(t.lam[i], t.d[i], t.n[i], t.grad[i], blocks), red);
+  if (threadIdx.x == 0) partial[(int64_t)i * RBLOCKS + blockIdx.x] = acc;
 }
 
 // Metric of the Poisson likelihood in data space, diag(1/lam) (SQRT = 0),
@@ -84,6 +175,21 @@ __global__ __launch_bounds__(RNT) void k_reduce(const double* __restrict__ parti
   for (int64_t k = threadIdx.x; k < n; k += RNT) acc += partial[k];
   acc = block_sum<RNT>(acc, red);
   if (threadIdx.x == 0) out[0] = acc;
+}
+
+// out[i] = the sum of array i's partials.
+struct SegBlocks {
+  int n[kReadoutSegs];
+};
+__global__ __launch_bounds__(RNT) void k_reduce_segments(const double* __restrict__ partial,
+                                                         SegBlocks blocks,
+                                                         double* __restrict__ out) {
+  __shared__ double red[RNT / 64];
+  const double* p = partial + (int64_t)blockIdx.x * RBLOCKS;
+  double acc = 0.0;
+  for (int64_t k = threadIdx.x; k < blocks.n[blockIdx.x]; k += RNT) acc += p[k];
+  acc = block_sum<RNT>(acc, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = acc;
 }
 
 // Cotangent of the metric's left square root J^T diag(lam^-1/2) at the base
@@ -284,11 +390,6 @@ int poisson_metric(int dtype, const void* lam, const void* t, int64_t n, int sqr
   return check_hip(hipGetLastError(), "poisson_metric");
 }
 
-// Blocks of the Poisson reduction for n elements: one partial per block.
-static int poisson_blocks(int64_t n) {
-  return (int)std::min<int64_t>(std::max<int64_t>((n + RNT - 1) / RNT, 1), RBLOCKS);
-}
-
 int poisson_nll_grad(int dtype, const void* lam, const void* d, int64_t n, double* nll,
                      void* grad, double* work, hipStream_t s) {
   const int blocks = poisson_blocks(n);
@@ -300,6 +401,65 @@ int poisson_nll_grad(int dtype, const void* lam, const void* d, int64_t n, doubl
                                              (double*)grad, work);
   k_reduce<<<1, RNT, 0, s>>>(work, blocks, nll);
   return check_hip(hipGetLastError(), "poisson_nll_grad");
+}
+
+template <typename T>
+static int poisson_segments_t(int64_t nseg, const void* const* lam, const void* const* d,
+                              const int64_t* n, double* nll, void* const* grad, double* work,
+                              hipStream_t s) {
+  for (int64_t i0 = 0; i0 < nseg; i0 += kReadoutSegs) {
+    const int m = (int)std::min<int64_t>(nseg - i0, kReadoutSegs);
+    PoissonSegs<T> t{};
+    SegBlocks b{};
+    int most = 1;
+    for (int i = 0; i < m; ++i) {
+      t.lam[i] = (const T*)lam[i0 + i];
+      t.d[i] = (const T*)d[i0 + i];
+      t.grad[i] = grad ? (T*)grad[i0 + i] : nullptr;
+      t.n[i] = n[i0 + i];
+      b.n[i] = poisson_blocks(t.n[i]);
+      most = std::max(most, b.n[i]);
+    }
+    double* w = work + i0 * RBLOCKS;
+    k_poisson_segments<T><<<dim3(most, m), RNT, 0, s>>>(t, w);
+    k_reduce_segments<<<m, RNT, 0, s>>>(w, b, nll + i0);
+  }
+  return check_hip(hipGetLastError(), "poisson_nll_grad_segments");
+}
+
+int poisson_nll_grad_segments(int dtype, int64_t nseg, const void* const* lam,
+                              const void* const* d, const int64_t* n, double* nll,
+                              void* const* grad, double* work, hipStream_t s) {
+  return dtype == 0 ? poisson_segments_t<float>(nseg, lam, d, n, nll, grad, work, s)
+                    : poisson_segments_t<double>(nseg, lam, d, n, nll, grad, work, s);
+}
+
+template <typename T, bool GATHER>
+static int readout_words_t(int64_t modules, const uint64_t* words, const int64_t* before,
+                           int64_t nwords, void* x, int64_t stride, void* const* v,
+                           hipStream_t s) {
+  using V = std::conditional_t<GATHER, T, const T>;
+  using X = std::conditional_t<GATHER, const T, T>;
+  const unsigned blocks = (unsigned)((nwords + kWords * (RNT / 64) - 1) / (kWords * (RNT / 64)));
+  for (int64_t i0 = 0; i0 < modules; i0 += kReadoutSegs) {
+    const int m = (int)std::min<int64_t>(modules - i0, kReadoutSegs);
+    ModulePtrs<V*> p{};
+    for (int i = 0; i < m; ++i) p.v[i] = (V*)v[i0 + i];
+    k_readout_words<T, GATHER><<<dim3(blocks, m), RNT, 0, s>>>(
+        words + i0 * nwords, before + i0 * nwords, nwords, (X*)x + i0 * stride, stride, p);
+  }
+  return check_hip(hipGetLastError(), GATHER ? "readout_gather_words" : "readout_scatter_words");
+}
+
+int readout_words(int dtype, bool gather, int64_t modules, const uint64_t* words,
+                  const int64_t* before, int64_t nwords, void* x, int64_t stride, void* const* v,
+                  hipStream_t s) {
+  if (modules <= 0 || nwords <= 0) return kOk;
+  if (dtype == 0)
+    return gather ? readout_words_t<float, true>(modules, words, before, nwords, x, stride, v, s)
+                  : readout_words_t<float, false>(modules, words, before, nwords, x, stride, v, s);
+  return gather ? readout_words_t<double, true>(modules, words, before, nwords, x, stride, v, s)
+                : readout_words_t<double, false>(modules, words, before, nwords, x, stride, v, s);
 }
 
 // ---------------------------------------------------------------- no-allocation variant

@@ -28,6 +28,15 @@ int poisson_metric(int dtype, const void* lam, const void* t, int64_t n, int sqr
                    void* out, hipStream_t s);
 int poisson_nll_grad(int dtype, const void* lam, const void* d, int64_t n, double* nll,
                      void* grad, double* work, hipStream_t s);
+// poisson_nll_grad of nseg arrays in one launch per 16: nll (nseg), ``work``
+// nseg kPoissonWorkDoubles doubles; grad NULL or an array of nseg pointers.
+int poisson_nll_grad_segments(int dtype, int64_t nseg, const void* const* lam,
+                              const void* const* d, const int64_t* n, double* nll,
+                              void* const* grad, double* work, hipStream_t s);
+// Read-out of several modules by bit words (gather), or its transpose.
+int readout_words(int dtype, bool gather, int64_t modules, const uint64_t* words,
+                  const int64_t* before, int64_t nwords, void* x, int64_t stride, void* const* v,
+                  hipStream_t s);
 // poisson_nll_grad with the partials in the library's static device scratch
 // (no allocation; calls that overlap on one GPU race on it).
 int poisson_nll_grad_noalloc(int dtype, const void* lam, const void* d, int64_t n, double* nll,

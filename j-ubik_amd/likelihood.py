@@ -5,6 +5,8 @@ erosita_likelihood.py:89).  Energy sum(lam - d log lam)
 metric diag(1/lam) and its left square root diag(lam^-1/2), composed with the
 linearisation of an amended forward.
 """
+import ctypes
+
 import torch
 
 from . import _device as dev
@@ -44,21 +46,32 @@ class Poissonian:
         leaves_d = _leaves(self.data)
         if len(leaves_l) != len(leaves_d):
             raise ValueError("lambda and data have different structure")
-        total = 0.0
-        grads = []
+        groups = {}  # element type -> the leaves of that type
+        parts = []
         for l, d in zip(leaves_l, leaves_d):
             dtype = dev.float_dtype(l)
             lt = dev.to_device(l, dtype).reshape(-1)
             dt = dev.to_device(d, dtype).reshape(-1)
             if lt.numel() != dt.numel():
                 raise ValueError("lambda and data sizes differ")
-            g = torch.empty_like(lt)
-            nll = torch.empty(1, dtype=torch.float64, device="cuda")
-            work = torch.empty(_lib.POISSON_WORK_BYTES // 8, dtype=torch.float64, device="cuda")
-            _lib.call("jubik_poisson_nll_grad", dev.code(dtype), dev.ptr(lt), dev.ptr(dt),
-                      lt.numel(), dev.ptr(nll), dev.ptr(g), dev.ptr(work), dev.stream())
-            total += float(nll.item())
-            grads.append(dev.like_input(g.reshape(tuple(l.shape)), l))
+            parts.append((lt, dt, torch.empty_like(lt)))
+            groups.setdefault(dtype, []).append(len(parts) - 1)
+        nll = torch.empty(len(parts), dtype=torch.float64, device="cuda")
+        work = torch.empty(len(parts) * (_lib.POISSON_WORK_BYTES // 8), dtype=torch.float64,
+                           device="cuda")
+        order = []  # leaf of every entry of nll
+        for dtype, members in groups.items():
+            lts, dts, gs = zip(*[parts[i] for i in members])
+            sizes = (ctypes.c_int64 * len(members))(*[t.numel() for t in lts])
+            _lib.call("jubik_poisson_nll_grad_segments", dev.code(dtype), len(members),
+                      dev.ptrs(lts), dev.ptrs(dts), sizes, dev.ptr(nll[len(order):]),
+                      dev.ptrs(gs), dev.ptr(work), dev.stream())
+            order += members
+        total = 0.0
+        for _, value in sorted(zip(order, nll.tolist())):
+            total += value
+        grads = [dev.like_input(g.reshape(tuple(l.shape)), l)
+                 for (_, _, g), l in zip(parts, leaves_l)]
         if isinstance(lam, Vector):
             return total, Vector(dict(zip(lam.tree.keys(), grads)))
         if isinstance(lam, dict):

@@ -2,8 +2,8 @@
 
 The builders keep the reference's host-side behaviour exactly (argument
 checks, in-place cut of the caller's array, key handling); the closures
-they return run as HIP kernels (broadcast multiply, gather by the C-order
-indices of the kept pixels).
+they return run as HIP kernels (broadcast multiply, gather of the kept pixels
+in C order).
 """
 import numpy as np
 import torch
@@ -69,14 +69,25 @@ def build_readout_function(flags, threshold=None, keys=None):
         keys = ['masked input']
     elif len(keys) != flags.shape[0]:
         raise ValueError("length of keys should match the number of flag maps.")
-    index_cache = {}
+    word_cache = {}
 
-    def _indices(i):
-        dkey = (i, torch.cuda.current_device())
-        if dkey not in index_cache:
-            flat = np.flatnonzero(~mask[i].reshape(-1)).astype(np.int64)
-            index_cache[dkey] = torch.as_tensor(flat, device="cuda")
-        return index_cache[dkey]
+    def _words():
+        """Kept pixels of the modules that are read out, on the current
+        device: bit words and kept pixels before each word, stacked (2,
+        modules, words), and the number of kept pixels per module."""
+        dkey = torch.cuda.current_device()
+        if dkey not in word_cache:
+            per = int(np.prod(mask.shape[1:]))
+            nwords = (per + 63) // 64
+            host = np.zeros((2, len(keys), nwords), dtype=np.int64)
+            for i in range(len(keys)):
+                bits = np.packbits(~mask[i].reshape(-1), bitorder="little")
+                host[0, i].view(np.uint8)[:bits.size] = bits
+            kept = np.cumsum(np.bitwise_count(host[0].view(np.uint64)), axis=1, dtype=np.int64)
+            host[1, :, 1:] = kept[:, :-1]
+            counts = kept[:, -1].tolist() if nwords else [0] * len(keys)
+            word_cache[dkey] = (torch.as_tensor(host, device="cuda"), counts)
+        return word_cache[dkey]
 
     def _apply_readout(x):
         if len(mask.shape) != 4:
@@ -86,18 +97,16 @@ def build_readout_function(flags, threshold=None, keys=None):
         dev.require_device()
         dtype = dev.float_dtype(x)
         xt = dev.to_device(x, dtype)
-        per = int(np.prod(xt.shape[1:]))
-        out = {}
-        for i, key in enumerate(keys):
-            idx = _indices(i)
-            v = torch.empty(idx.numel(), dtype=dtype, device="cuda")
-            src = xt[i].reshape(-1)
-            if src.numel() != per:
-                raise ValueError("input module shape does not match the flags")
-            _lib.call("jubik_readout_gather", dev.code(dtype), dev.ptr(src), dev.ptr(idx),
-                      idx.numel(), dev.ptr(v), dev.stream())
-            out[key] = dev.like_input(v, x)
-        return Vector(out)
+        per, pixels = int(np.prod(xt.shape[1:])), int(np.prod(mask.shape[1:]))
+        if xt.shape[0] < len(keys):
+            raise IndexError("input has fewer modules than there are keys")
+        if per < pixels:
+            raise ValueError("input module shape does not match the flags")
+        words, counts = _words()
+        out = [torch.empty(c, dtype=dtype, device="cuda") for c in counts]
+        _lib.call("jubik_readout_gather_words", dev.code(dtype), len(keys), dev.ptr(words[0]),
+                  dev.ptr(words[1]), pixels, dev.ptr(xt), per, dev.ptrs(out), dev.stream())
+        return Vector({key: dev.like_input(v, x) for key, v in zip(keys, out)})
 
     def _transpose(vec, like_shape=None):
         """Scatter read-out vectors back into a zero (M, E, H, W) array."""
@@ -105,14 +114,16 @@ def build_readout_function(flags, threshold=None, keys=None):
         shape = mask.shape
         first = vec[keys[0]]
         dtype = dev.float_dtype(first)
-        out = torch.empty(shape, dtype=dtype, device="cuda")
-        per = int(np.prod(shape[1:]))
-        for i, key in enumerate(keys):
-            idx = _indices(i)
-            v = dev.to_device(vec[key], dtype)
-            dst = out[i].reshape(-1)
-            _lib.call("jubik_readout_scatter", dev.code(dtype), dev.ptr(v), dev.ptr(idx),
-                      idx.numel(), per, dev.ptr(dst), dev.stream())
+        words, counts = _words()
+        vs = [dev.to_device(vec[key], dtype) for key in keys]
+        if any(v.numel() < c for v, c in zip(vs, counts)):
+            raise ValueError("read-out vectors are shorter than the kept pixels")
+        # modules that are not read out stay zero
+        new = torch.empty if len(keys) == shape[0] else torch.zeros
+        out = new(shape, dtype=dtype, device="cuda")
+        _lib.call("jubik_readout_scatter_words", dev.code(dtype), len(keys), dev.ptr(words[0]),
+                  dev.ptr(words[1]), int(np.prod(shape[1:])), dev.ptrs(vs), dev.ptr(out),
+                  dev.stream())
         return dev.like_input(out, first)
 
     _apply_readout.transpose = _transpose
