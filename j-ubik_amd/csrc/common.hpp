@@ -165,14 +165,8 @@ __device__ __forceinline__ T tent_weight(int d, double step, int t) {
 }
 __device__ __forceinline__ double tent_step(int d) { return d > 1 ? 1.0 / (d - 1) : 0.0; }
 
-// Streaming access to workspace arrays that are written once and read once
-// by the next pass: non-temporal loads and stores.
-template <typename T>
-__device__ __forceinline__ cplx<T> ld_stream(const cplx<T>* p) {
-  typedef T v2 __attribute__((ext_vector_type(2)));
-  const v2 v = __builtin_nontemporal_load(reinterpret_cast<const v2*>(p));
-  return cplx<T>{v.x, v.y};
-}
+// Streaming stores to workspace arrays that are written once and read once by
+// the next pass: non-temporal.
 template <typename T>
 __device__ __forceinline__ void st_stream(cplx<T>* p, cplx<T> c) {
   typedef T v2 __attribute__((ext_vector_type(2)));
@@ -215,6 +209,13 @@ __device__ __forceinline__ T gather_load(const Gather& g, int off) {
     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(g.r, off, 0, 0));
 }
 
+template <typename T>
+__device__ __forceinline__ T buffer_load_real(__amdgpu_buffer_rsrc_t r, int off, int uniform = 0) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, uniform, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, uniform, 0));
+}
 template <typename T, int AUX = 0>
 __device__ __forceinline__ cplx<T> buffer_load(__amdgpu_buffer_rsrc_t r, int off, int uniform = 0) {
   if constexpr (sizeof(T) == 4)
@@ -265,11 +266,11 @@ struct RowAccess {
     return buffer_load<T, AUX>(r, off, step * ROW);
   }
   template <int AUX = 0>
-  __device__ __forceinline__ void store(int off, cplx<T> v) const {
+  __device__ __forceinline__ void store(int off, cplx<T> v, int step = 0) const {
     if constexpr (sizeof(T) == 4)
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, off, 0, AUX);
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, off, step * ROW, AUX);
     else
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, off, 0, AUX);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, off, step * ROW, AUX);
   }
 };
 

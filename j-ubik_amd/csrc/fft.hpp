@@ -389,24 +389,25 @@ __host__ __device__ constexpr int lds_stride(int L, int V) {
 }
 
 // Threads per work-group of a pass over V vectors of length L that keeps
-// every value in registers from stage to stage (plan kind 0): the multiple of
+// every value in registers from stage to stage (plan kind pl): the multiple of
 // 64 whose stages issue the fewest butterfly points, idle lanes counted, with
 // at most max_points values per thread and stage; among equals the one that
 // holds fewer values.
-__host__ __device__ constexpr int stage_points(int L, int V, int nt, int s) {
-  const int R = plan_radix(L, s);
+__host__ __device__ constexpr int stage_points(int L, int V, int nt, int s, int pl) {
+  const int R = plan_radix(L, s, pl);
   return ((V * (L / R) + nt - 1) / nt) * R;
 }
-__host__ __device__ constexpr int register_threads(int L, int V, int max_points) {
+__host__ __device__ constexpr int register_threads(int L, int V, int max_points,
+                                                  int pl = 0) {
   for (int most_nt = 256; most_nt <= 512; most_nt += 256) {
     int best = 0, best_cost = 0, best_most = 0;
     for (int nt = 64; nt <= most_nt; nt += 64) {
       int cost = 0, most = 0, radix = 0;
-      for (int s = 0; s < plan_stages(L); ++s) {
-        const int q = stage_points(L, V, nt, s);
+      for (int s = 0; s < plan_stages(L, pl); ++s) {
+        const int q = stage_points(L, V, nt, s, pl);
         cost += q * nt;
         most = q > most ? q : most;
-        radix = plan_radix(L, s) > radix ? plan_radix(L, s) : radix;
+        radix = plan_radix(L, s, pl) > radix ? plan_radix(L, s, pl) : radix;
       }
       if (most > max_points && most > radix) continue;
       if (best == 0 || cost < best_cost || (cost == best_cost && most < best_most)) {
@@ -430,6 +431,23 @@ __host__ __device__ constexpr int split_stride(int L, int V, int elem) {
   const int per = slots / V > 8 ? slots / V : 8;
   const int r = (V >= 16 ? 16 : per) + 1;
   return L + ((r - L % slots) % slots + slots) % slots;
+}
+
+// Marks values that idle lanes leave unwritten as free inside a loop: without
+// it they stay alive, in registers, from one turn to the next.
+template <typename T>
+__device__ __forceinline__ void forget(T& v) {
+  v = __builtin_nondeterministic_value(v);
+}
+template <typename T>
+__device__ __forceinline__ void forget(cplx<T>& v) {
+  forget(v.re);
+  forget(v.im);
+}
+template <typename T, int N>
+__device__ __forceinline__ void forget(T (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) forget(v[i]);
 }
 
 // ---------------------------------------------------------------- stages
