@@ -223,6 +223,20 @@ __device__ __forceinline__ cplx<T> buffer_load(__amdgpu_buffer_rsrc_t r, int off
   else
     return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b128(r, off, uniform, AUX));
 }
+// v = entry e of a table of L twiddles, if there is one.  In FP64 through a
+// buffer resource (zero past the table): a 16-byte load under a branch is
+// compiled through scratch memory (L = 320 at 512^2 x 2E, the six PSF passes
+// 94 -> 82 us); in FP32 the branch costs fewer registers.
+template <int L, typename T>
+__device__ __forceinline__ void load_root(cplx<T>& v, const cplx<T>* table, int e) {
+  constexpr int B = (int)sizeof(cplx<T>);
+  if constexpr (sizeof(T) == 8)
+    v = buffer_load<T>(
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<cplx<T>*>(table), 0, L * B, 0x00020000),
+        e * B);
+  else if (e < L)
+    v = table[e];
+}
 constexpr int kStream = 2;                     // cache policy: non-temporal
 constexpr int kOutOfRange = (int)0x80000000;  // lies past every range
 
@@ -321,6 +335,24 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   constexpr int kXcds = 8;
   if (nb % kXcds) return b;
   return (b % kXcds) * (nb / kXcds) + b / kXcds;
+}
+
+// Sum over a wave, in lane 63, by data-parallel moves between lanes: no trip
+// through the LDS per step, where a shuffle of a double takes two.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, ROWS, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: sums of rows of 16 lanes
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  return dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
 }
 
 // Block-wide sum of one double per thread (NT a multiple of 64).
