@@ -165,8 +165,14 @@ __device__ __forceinline__ T tent_weight(int d, double step, int t) {
 }
 __device__ __forceinline__ double tent_step(int d) { return d > 1 ? 1.0 / (d - 1) : 0.0; }
 
-// Streaming stores to workspace arrays that are written once and read once by
-// the next pass: non-temporal.
+// Streaming access to workspace arrays that are written once and read once
+// by the next pass: non-temporal loads and stores.
+template <typename T>
+__device__ __forceinline__ cplx<T> ld_stream(const cplx<T>* p) {
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  const v2 v = __builtin_nontemporal_load(reinterpret_cast<const v2*>(p));
+  return cplx<T>{v.x, v.y};
+}
 template <typename T>
 __device__ __forceinline__ void st_stream(cplx<T>* p, cplx<T> c) {
   typedef T v2 __attribute__((ext_vector_type(2)));
@@ -303,15 +309,14 @@ struct Tile {
   static constexpr int V = tile_vectors(JUBIK_COL_TILE_BYTES, L, (int)sizeof(cplx<T>));
 };
 
-// Column passes of the PSF operator: a tile of 128 bytes of every spectrum
-// row (one cache line: 16 float or 8 double columns), at most the L/2 stored
-// columns, whatever its length.  A half line per row is slower even where it
-// lets more work-groups share a CU (FP32, L = 432 in fold mode at 1024^2 x 4E,
-// forward / adjoint: 8 columns 186 / 168, 16 columns 162 / 140 us).  Two lines
-// pay at L = 192 in FP64 only, whose one-line work-group would be two waves
-// that the LDS keeps few of (512^2 x 4E: 42 / 39 against 37 / 35 us).
+// Column passes of the PSF operator.  FP64: a tile of 128 bytes of every
+// spectrum row (one cache line, 8 columns), at most the L/2 stored columns,
+// whatever its length.  Two lines pay at L = 192 only, whose one-line
+// work-group would be two waves that the LDS keeps few of (512^2 x 4E: 42 / 39
+// against 37 / 35 us).  FP32: Tile (lp_cols_f32).
 __host__ __device__ constexpr int col_vectors(int L, int elem) {
-  int v = elem == 16 && L == 192 ? 16 : 128 / elem;
+  if (elem == 8) return tile_vectors(JUBIK_COL_TILE_BYTES, L, elem);
+  int v = L == 192 ? 16 : 8;
   while (v > 8 && v / 2 >= L / 2) v /= 2;
   return v;
 }

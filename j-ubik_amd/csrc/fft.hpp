@@ -111,8 +111,13 @@ struct RootTable {
 template <int N>
 inline constexpr RootTable<N> kRoots{};
 
+// In a sum of two products that is contracted to a multiply-add one product is
+// rounded, and which one is up to the order the compiler gives the sum.  FIXED
+// writes it out where that order differed between kernels of one length: the
+// sums of radix 7 and of the twiddles of radix 14 (the grids 567 and 1134).
+//
 // x * W_N^e (conjugated for the inverse); e is a constant after unrolling.
-template <typename T, int N, bool INV>
+template <typename T, int N, bool INV, bool FIXED = false>
 __device__ __forceinline__ cplx<T> twiddle_c(cplx<T> x, int e) {
   if (e == 0) return x;
   if (4 * e == N) return mul_mi<T, INV>(x);
@@ -120,6 +125,7 @@ __device__ __forceinline__ cplx<T> twiddle_c(cplx<T> x, int e) {
   if (4 * e == 3 * N) return mul_mi<T, !INV>(x);
   const T wr = T(kRoots<N>.re[e]);
   const T wi = INV ? T(-kRoots<N>.im[e]) : T(kRoots<N>.im[e]);
+  if (FIXED && N == 14 && !INV && e < 4) return {T(fma(x.im, -wi, x.re * wr)), x.re * wi + x.im * wr};
   return {x.re * wr - x.im * wi, x.re * wi + x.im * wr};
 }
 
@@ -210,6 +216,7 @@ struct Dft<T, 5, INV> {
 
 template <typename T, bool INV>
 struct Dft<T, 7, INV> {
+  template <bool FIXED = false>
   static __device__ __forceinline__ void run(cplx<T>* v) {
     const T c1 = T(0.62348980185873353052500488400424);
     const T c2 = T(-0.22252093395631440428890256449679);
@@ -230,8 +237,11 @@ struct Dft<T, 7, INV> {
     cplx<T> m3 = {x0.re + c3 * a1.re + c1 * a2.re + c2 * a3.re,
                   x0.im + c3 * a1.im + c1 * a2.im + c2 * a3.im};
     // sin(2 pi t q / 7) for (q,t): q=1: s1 s2 s3; q=2: s2 -s3 -s1; q=3: s3 -s1 s2
-    cplx<T> n1 = mul_mi<T, INV>(cplx<T>{s1 * b1.re + s2 * b2.re + s3 * b3.re,
-                                        s1 * b1.im + s2 * b2.im + s3 * b3.im});
+    auto sum1 = [&](T x1, T x2, T x3) -> T {
+      if constexpr (FIXED) return fma(s3, x3, fma(s2, x2, s1 * x1));
+      else return s1 * x1 + s2 * x2 + s3 * x3;
+    };
+    cplx<T> n1 = mul_mi<T, INV>(cplx<T>{sum1(b1.re, b2.re, b3.re), sum1(b1.im, b2.im, b3.im)});
     cplx<T> n2 = mul_mi<T, INV>(cplx<T>{s2 * b1.re - s3 * b2.re - s1 * b3.re,
                                         s2 * b1.im - s3 * b2.im - s1 * b3.im});
     cplx<T> n3 = mul_mi<T, INV>(cplx<T>{s3 * b1.re - s1 * b2.re + s2 * b3.re,
@@ -255,16 +265,21 @@ __host__ __device__ constexpr int dft_split(int N) {
   return N % 4 == 0 ? 4 : N % 2 == 0 ? 2 : N % 3 == 0 ? 3 : N % 5 == 0 ? 5 : 7;
 }
 
-template <typename T, int N, bool INV, bool BASE = dft_is_base(N)>
+template <typename T, int N, bool INV, bool FIXED = false, bool BASE = dft_is_base(N)>
 struct RegDft;
 
-template <typename T, int N, bool INV>
-struct RegDft<T, N, INV, true> {
-  static __device__ __forceinline__ void run(cplx<T>* v) { Dft<T, N, INV>::run(v); }
+template <typename T, int N, bool INV, bool FIXED>
+struct RegDft<T, N, INV, FIXED, true> {
+  static __device__ __forceinline__ void run(cplx<T>* v) {
+    if constexpr (N == 7)
+      Dft<T, 7, INV>::template run<FIXED>(v);
+    else
+      Dft<T, N, INV>::run(v);
+  }
 };
 
-template <typename T, int N, bool INV>
-struct RegDft<T, N, INV, false> {
+template <typename T, int N, bool INV, bool FIXED>
+struct RegDft<T, N, INV, FIXED, false> {
   static constexpr int A = dft_split(N);
   static constexpr int B = N / A;
   static __device__ __forceinline__ void run(cplx<T>* v) {
@@ -274,17 +289,17 @@ struct RegDft<T, N, INV, false> {
 #pragma unroll
       for (int j = 0; j < B; ++j) u[i][j] = v[i + A * j];
 #pragma unroll
-    for (int i = 0; i < A; ++i) RegDft<T, B, INV>::run(u[i]);
+    for (int i = 0; i < A; ++i) RegDft<T, B, INV, FIXED>::run(u[i]);
 #pragma unroll
     for (int i = 1; i < A; ++i)
 #pragma unroll
-      for (int k = 1; k < B; ++k) u[i][k] = twiddle_c<T, N, INV>(u[i][k], i * k);
+      for (int k = 1; k < B; ++k) u[i][k] = twiddle_c<T, N, INV, FIXED>(u[i][k], i * k);
 #pragma unroll
     for (int k = 0; k < B; ++k) {
       cplx<T> w[A];
 #pragma unroll
       for (int i = 0; i < A; ++i) w[i] = u[i][k];
-      RegDft<T, A, INV>::run(w);
+      RegDft<T, A, INV, FIXED>::run(w);
 #pragma unroll
       for (int q = 0; q < A; ++q) v[k + B * q] = w[q];
     }
@@ -390,15 +405,15 @@ __host__ __device__ constexpr int lds_stride(int L, int V) {
 
 // Threads per work-group of a pass over V vectors of length L that keeps
 // every value in registers from stage to stage (plan kind pl): the multiple of
-// 64 whose stages issue the fewest butterfly points, idle lanes counted, with
-// at most max_points values per thread and stage; among equals the one that
-// holds fewer values.
+// 64 up to 256, or else up to 512, whose stages issue the fewest butterfly
+// points, idle lanes counted, with no more values per thread and stage than
+// the longest butterfly has; among equals the one that holds fewer values.
+// 512 where a thread has to hold more.
 __host__ __device__ constexpr int stage_points(int L, int V, int nt, int s, int pl) {
   const int R = plan_radix(L, s, pl);
   return ((V * (L / R) + nt - 1) / nt) * R;
 }
-__host__ __device__ constexpr int register_threads(int L, int V, int max_points,
-                                                  int pl = 0) {
+__host__ __device__ constexpr int register_threads(int L, int V, int pl = 0) {
   for (int most_nt = 256; most_nt <= 512; most_nt += 256) {
     int best = 0, best_cost = 0, best_most = 0;
     for (int nt = 64; nt <= most_nt; nt += 64) {
@@ -409,7 +424,7 @@ __host__ __device__ constexpr int register_threads(int L, int V, int max_points,
         most = q > most ? q : most;
         radix = plan_radix(L, s, pl) > radix ? plan_radix(L, s, pl) : radix;
       }
-      if (most > max_points && most > radix) continue;
+      if (most > radix) continue;
       if (best == 0 || cost < best_cost || (cost == best_cost && most < best_most)) {
         best = nt;
         best_cost = cost;
@@ -448,6 +463,19 @@ template <typename T, int N>
 __device__ __forceinline__ void forget(T (&v)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) forget(v[i]);
+}
+
+// Values that the compiler knows nothing about: a butterfly of them is
+// contracted (and so rounded) as one of values that a loop left.
+template <typename T>
+__device__ __forceinline__ void opaque(cplx<T>& v) {
+  asm volatile("" : "+v"(v.re));
+  asm volatile("" : "+v"(v.im));
+}
+template <typename T, int N>
+__device__ __forceinline__ void opaque(T (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) opaque(v[i]);
 }
 
 // ---------------------------------------------------------------- stages
@@ -504,7 +532,7 @@ struct Stage {
             v[b][t] = INV ? cmulc(v[b][t], w) : cmul(v[b][t], w);
           }
         }
-        RegDft<T, R, INV>::run(v[b]);
+        RegDft<T, R, INV, L % 567 == 0>::run(v[b]);
       }
     }
   }

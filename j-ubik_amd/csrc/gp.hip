@@ -24,11 +24,22 @@ constexpr int GNT = 256;
 // (measured at N = 1024: forward 15.4 -> 13.0 us; the column pass is faster
 // at 256).
 constexpr int GNR = 512;
+constexpr int kCus = 256;  // compute units of the chip
+
+// Tiles of the column pass in LDS: a tile's width is at most N; the adjoint
+// (MODE 1) gathers uplanes cotangent planes per column and runs at half the
+// width, twice the work-groups.
+template <typename T, int N, int MODE = 0>
+struct GpLdsTile {
+  static constexpr int V0 = Tile<T, N>::V < N ? Tile<T, N>::V : N;
+  static constexpr int V = (MODE == 1 && V0 > 2) ? V0 / 2 : V0;
+};
 
 // Tiles of the column pass: 8 (wide) or 4 FP32 columns, half as many in FP64.
 // A work-group keeps its tile in registers, loaded straight into the first
-// stage and stored from the last, with one butterfly per thread and stage; the
-// LDS holds one component at a time.  The pass is bound by the latency of one
+// stage and stored from the last; up to 512 threads hold one butterfly each (N =
+// 567), or a few short ones (2048 wide: two of 16 points, four of 8); the LDS
+// holds one component at a time.  The pass is bound by the latency of one
 // tile where the grid gives a work-group or less per CU, and by the partial
 // lines of its rows where it gives many.  us per launch, forward / adjoint,
 // LDS-resident tiles of 52 KiB before -> now: N = 2048 x 4 samples 228 / 97 ->
@@ -41,7 +52,7 @@ template <typename T, int N, bool WIDE>
 struct GpTile {
   static constexpr int V = (WIDE ? 32 : 16) / (int)sizeof(T);
   static constexpr int PL = 1;
-  static constexpr int NT = register_threads(N, V, 0, PL);
+  static constexpr int NT = register_threads(N, V, PL);
 };
 
 // amp * xi, rounded: contracted into the first butterfly's sums, a field's
@@ -165,6 +176,7 @@ __global__ __launch_bounds__((GpTile<T, N, WIDE>::NT)) void gp_cols(
     const int e = tid + i * NT;
     if (e < N) tw[e] = twr[i];
   }
+  if constexpr (MODE == 2 && N == 2048) opaque(v0);  // else it rounds unlike MODE 1
   F0::compute(v0, tw, tid);
   const RowAccess<T, N> out(Tw + smp * N * N, N);
   auto store = [&](auto stage, auto& regs) {
@@ -192,6 +204,197 @@ __global__ __launch_bounds__((GpTile<T, N, WIDE>::NT)) void gp_cols(
       F2::compute(v2, tw, tid);
       store(F2{}, v2);
     }
+  }
+}
+
+// The same pass on the small grids (N <= 256), with the tile in LDS and large
+// radices in its forward: one or two rounds of work-groups either way.  It
+// rounds as the products of the metric have to (see lp_cols_f32).
+template <typename T, int N, int MODE>
+__global__ __launch_bounds__(GNT) void gp_cols_lds(GpGeom g, const T* __restrict__ amp_ref,
+                                               const T* __restrict__ amp_alpha,
+                                               const T* __restrict__ xi_ref,
+                                               const T* __restrict__ xi_alpha,
+                                               const T* __restrict__ u,
+                                               const T* __restrict__ dnu,
+                                               const cplx<T>* __restrict__ twg,
+                                               cplx<T>* __restrict__ Tw) {
+  constexpr int V = GpLdsTile<T, N, MODE>::V;
+  constexpr int VS = lds_stride(N, V);
+  __shared__ cplx<T> buf[V * VS];
+  __shared__ cplx<T> tw[N];
+  const int tid = threadIdx.x;
+  const int c0 = xcd_tile(blockIdx.x, gridDim.x) * V;
+  const int64_t smp = blockIdx.y;
+  if (xi_ref) xi_ref += smp * N * N;
+  if (xi_alpha) xi_alpha += smp * N * N;
+  if (u) u += smp * g.uplanes * g.H * g.W * (g.ucomplex ? 2 : 1);
+  Tw += smp * N * N;
+  // Loads are issued in unrolled chunks of CH elements per thread (their
+  // latencies overlap), twiddles first.
+  constexpr int TPT = (N + GNT - 1) / GNT;
+  cplx<T> twr[TPT];
+#pragma unroll
+  for (int u2 = 0; u2 < TPT; ++u2) {
+    const int e = tid + u2 * GNT;
+    if (e < N) twr[u2] = twg[e];
+  }
+  constexpr int EPT = (V * N + GNT - 1) / GNT;
+  constexpr int CH = (MODE == 0 ? 16 : 8) / (sizeof(T) / 4);
+  constexpr int CHK = EPT < CH ? EPT : CH;
+  // MODE 1 reads the planes through zero-reading gathers (elements outside
+  // the sky grid read zero), one buffer resource per plane (so offsets stay
+  // 32-bit however many planes), planes outer and the chunk unrolled inside,
+  // so a chunk's loads of one plane are in flight together.
+  const int64_t plane = (int64_t)g.H * g.W;
+  const int64_t nn = MODE == 0 ? (int64_t)N * N : 0;
+  const Gather gar = make_gather(amp_ref, nn), gxr = make_gather(xi_ref, nn);
+  const Gather gaa = make_gather(amp_alpha, g.has_alpha ? nn : 0);
+  const Gather gxa = make_gather(xi_alpha, g.has_alpha ? nn : 0);
+  // Row-vector gathers: the tile's V adjacent columns of a row are one 8- or
+  // 16-byte load per array, V times fewer loads than one per element (the
+  // adjoint's planes need W to be a multiple of V, so that a tile lies wholly
+  // inside or wholly outside the sky grid).  Same products and sums per
+  // element as the per-element path below.
+  constexpr bool kRowVec = (V * sizeof(T) == 8 || V * sizeof(T) == 16) && N % V == 0;
+  // complex planes: a row of the tile is V complex values
+  constexpr bool kRowVecC = 2 * V * sizeof(T) == 16 && N % V == 0;
+  bool row_vec = false;
+  if constexpr (kRowVec) {
+    row_vec = MODE == 0 || (g.W % V == 0 && (!g.ucomplex || kRowVecC));
+    if (row_vec) {
+      using VT = T __attribute__((ext_vector_type(V)));
+      constexpr int RPT = (N + GNT - 1) / GNT;  // rows per thread
+      constexpr int CR = RPT < 4 ? RPT : 4;     // rows per chunk
+      for (int r0 = 0; r0 < RPT; r0 += CR) {
+        VT va[CR], vb[CR];
+#pragma unroll
+        for (int c = 0; c < CR; ++c) {
+          const int x1 = tid + (r0 + c) * GNT;
+          if constexpr (MODE == 0) {
+            const bool ok = x1 < N;
+            const int o = x1 * N + c0;
+            const int orf = gather_off<T>(gar, ok, o);
+            const int oal = gather_off<T>(gaa, ok && g.has_alpha, o);
+            va[c] = gather_load<VT>(gar, orf) * gather_load<VT>(gxr, orf);
+            vb[c] = gather_load<VT>(gaa, oal) * gather_load<VT>(gxa, oal);
+          } else {
+            va[c] = VT(T(0));
+            vb[c] = VT(T(0));
+          }
+        }
+        if constexpr (MODE == 1) {
+          if (g.ucomplex) {
+            if constexpr (kRowVecC) {
+              using VT2 = T __attribute__((ext_vector_type(2 * V)));
+              for (int pl = 0; pl < g.uplanes; ++pl) {
+                const cplx<T>* up = reinterpret_cast<const cplx<T>*>(u) + pl * plane;
+                const Gather gu = make_gather(up, plane);
+#pragma unroll
+                for (int c = 0; c < CR; ++c) {
+                  const int x1 = tid + (r0 + c) * GNT;
+                  const bool ok = x1 < g.H && c0 < g.W;
+                  const VT2 w =
+                      gather_load<VT2>(gu, gather_off<cplx<T>>(gu, ok, x1 * g.W + c0));
+#pragma unroll
+                  for (int v = 0; v < V; ++v) {
+                    va[c][v] += w[2 * v];
+                    vb[c][v] += w[2 * v + 1];
+                  }
+                }
+              }
+            }
+          } else {
+            for (int pl = 0; pl < g.uplanes; ++pl) {
+              const Gather gu = make_gather(u + pl * plane, plane);
+              const T dn = g.has_alpha ? dnu[pl % g.E] : T(0);
+#pragma unroll
+              for (int c = 0; c < CR; ++c) {
+                const int x1 = tid + (r0 + c) * GNT;
+                const bool ok = x1 < g.H && c0 < g.W;
+                const VT uv = gather_load<VT>(gu, gather_off<T>(gu, ok, x1 * g.W + c0));
+                va[c] += uv;
+                vb[c] += dn * uv;
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < CR; ++c) {
+          const int x1 = tid + (r0 + c) * GNT;
+          if (x1 < N) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) buf[v * VS + x1] = cplx<T>{va[c][v], vb[c][v]};
+          }
+        }
+      }
+    }
+  }
+  for (int u0 = 0; !row_vec && u0 < EPT; u0 += CHK) {
+    cplx<T> val[CHK];
+#pragma unroll
+    for (int c = 0; c < CHK; ++c) val[c] = cplx<T>{T(0), T(0)};
+    if constexpr (MODE == 0) {
+      // Zero-reading gathers (the alpha field reads zero when absent): the
+      // chunk's loads of all four arrays are in flight together.
+#pragma unroll
+      for (int c = 0; c < CHK; ++c) {
+        const int e = tid + (u0 + c) * GNT;
+        const int x1 = e / V, v = e - (e / V) * V;
+        const int x2 = c0 + v;
+        const bool ok = (V * N % GNT == 0 || e < V * N) && (N % V == 0 || x2 < N);
+        const int o = x1 * N + x2;
+        const int orf = gather_off<T>(gar, ok, o), oal = gather_off<T>(gaa, ok && g.has_alpha, o);
+        val[c].re = gather_load<T>(gar, orf) * gather_load<T>(gxr, orf);
+        val[c].im = gather_load<T>(gaa, oal) * gather_load<T>(gxa, oal);
+      }
+    } else if (g.ucomplex) {
+      for (int pl = 0; pl < g.uplanes; ++pl) {
+        const cplx<T>* up = reinterpret_cast<const cplx<T>*>(u) + pl * plane;
+        const Gather gu = make_gather(up, plane);
+#pragma unroll
+        for (int c = 0; c < CHK; ++c) {
+          const int e = tid + (u0 + c) * GNT;
+          const int x1 = e / V, v = e - (e / V) * V;
+          const int x2 = c0 + v;
+          const bool ok = (V * N % GNT == 0 || e < V * N) && x1 < g.H && x2 < g.W;
+          val[c] = cadd(val[c], gather_load<cplx<T>>(gu, gather_off<cplx<T>>(gu, ok, x1 * g.W + x2)));
+        }
+      }
+    } else {
+      for (int pl = 0; pl < g.uplanes; ++pl) {
+        const Gather gu = make_gather(u + pl * plane, plane);
+        const T dn = g.has_alpha ? dnu[pl % g.E] : T(0);
+#pragma unroll
+        for (int c = 0; c < CHK; ++c) {
+          const int e = tid + (u0 + c) * GNT;
+          const int x1 = e / V, v = e - (e / V) * V;
+          const int x2 = c0 + v;
+          const bool ok = (V * N % GNT == 0 || e < V * N) && x1 < g.H && x2 < g.W;
+          const T uv = gather_load<T>(gu, gather_off<T>(gu, ok, x1 * g.W + x2));
+          val[c].re += uv;
+          val[c].im += dn * uv;
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CHK; ++c) {
+      const int e = tid + (u0 + c) * GNT;
+      if (e >= V * N) continue;
+      const int x1 = e / V, v = e - (e / V) * V;
+      buf[v * VS + x1] = val[c];
+    }
+  }
+#pragma unroll
+  for (int u2 = 0; u2 < TPT; ++u2) {
+    const int e = tid + u2 * GNT;
+    if (e < N) tw[e] = twr[u2];
+  }
+  __syncthreads();
+  fft_lds<T, N, V, VS, GNT, false, kFewVectorPlan<N, V, GNT>>(buf, tw, tid);
+  for (int e = tid; e < V * N; e += GNT) {
+    const int x1 = e / V, v = e - (e / V) * V;
+    if (N % V == 0 || c0 + v < N) Tw[(int64_t)x1 * N + c0 + v] = buf[v * VS + x1];
   }
 }
 
@@ -371,6 +574,12 @@ template <typename T, int N>
 struct GpOps {
   using C = cplx<T>;
   // Column pass over S samples: launch(wide, tiles, threads).
+  // The small FP32 grids run the column pass in LDS (gp_cols_lds).
+  static constexpr bool kLds = std::is_same<T, float>::value && N <= 256;
+  template <int MODE>
+  static dim3 lds_tiles(int S) {
+    return dim3((N + GpLdsTile<T, N, MODE>::V - 1) / GpLdsTile<T, N, MODE>::V, S);
+  }
   template <class F>
   static void with_tile(int S, F&& launch) {
     auto go = [&](auto wide) {
@@ -383,7 +592,7 @@ struct GpOps {
     // 34 us, 567 in FP64 13.4 / 19.2 us, 2048 x 4 samples 120 / 139 us, 256 x 32
     // samples 12.5 / 14.3 us, but 1024 17.2 / 15.0 us and 512 7.1 / 6.7 us).
     constexpr int wide_tiles = (N + GpTile<T, N, true>::V - 1) / GpTile<T, N, true>::V;
-    if (N * sizeof(T) % 128 != 0 || (int64_t)wide_tiles * S >= 256)
+    if (N * sizeof(T) % 128 != 0 || (int64_t)wide_tiles * S >= kCus)
       go(std::true_type{});
     else
       go(std::false_type{});
@@ -393,11 +602,16 @@ struct GpOps {
                      const void* dnu, void* sky, hipStream_t s) {
     {
       TimedLaunch _t("gp_cols_fwd", s);
-      with_tile(g.S, [&](auto wide, dim3 grid, int threads) {
-        gp_cols<T, N, 0, decltype(wide)::value><<<grid, threads, 0, s>>>(
+      if constexpr (kLds)
+        gp_cols_lds<T, N, 0><<<lds_tiles<0>(g.S), GNT, 0, s>>>(
             g, (const T*)amp_ref, (const T*)amp_alpha, (const T*)xi_ref, (const T*)xi_alpha,
             nullptr, nullptr, (const C*)b.tw, (C*)b.work);
-      });
+      else
+        with_tile(g.S, [&](auto wide, dim3 grid, int threads) {
+          gp_cols<T, N, 0, decltype(wide)::value><<<grid, threads, 0, s>>>(
+              g, (const T*)amp_ref, (const T*)amp_alpha, (const T*)xi_ref, (const T*)xi_alpha,
+              nullptr, nullptr, (const C*)b.tw, (C*)b.work);
+        });
     }
     {
       TimedLaunch _t("gp_rows_fwd", s);
@@ -412,11 +626,17 @@ struct GpOps {
                      const void* dnu, const void* sky, void* dsky, hipStream_t s) {
     {
       TimedLaunch _t("gp_cols_fwd", s);
-      with_tile(g.work_shared ? 1 : g.S, [&](auto wide, dim3 grid, int threads) {
-        gp_cols<T, N, 0, decltype(wide)::value><<<grid, threads, 0, s>>>(
+      const int S = g.work_shared ? 1 : g.S;
+      if constexpr (kLds)
+        gp_cols_lds<T, N, 0><<<lds_tiles<0>(S), GNT, 0, s>>>(
             g, (const T*)amp_ref, (const T*)amp_alpha, (const T*)v_ref, (const T*)v_alpha, nullptr,
             nullptr, (const C*)b.tw, (C*)b.work);
-      });
+      else
+        with_tile(S, [&](auto wide, dim3 grid, int threads) {
+          gp_cols<T, N, 0, decltype(wide)::value><<<grid, threads, 0, s>>>(
+              g, (const T*)amp_ref, (const T*)amp_alpha, (const T*)v_ref, (const T*)v_alpha,
+              nullptr, nullptr, (const C*)b.tw, (C*)b.work);
+        });
     }
     {
       TimedLaunch _t("gp_rows_tangent", s);
@@ -431,17 +651,22 @@ struct GpOps {
                        void* g_alpha, hipStream_t s, GpHyper hy) {
     {
       TimedLaunch _t("gp_cols_adj", s);
-      with_tile(g.S, [&](auto wide, dim3 grid, int threads) {
-        constexpr bool W = decltype(wide)::value;
-        if (g.ucomplex && g.uplanes == 1)
-          gp_cols<T, N, 2, W><<<grid, threads, 0, s>>>(g, nullptr, nullptr, nullptr, nullptr,
-                                                      (const T*)u, nullptr, (const C*)b.tw,
-                                                      (C*)b.work);
-        else
-          gp_cols<T, N, 1, W><<<grid, threads, 0, s>>>(g, nullptr, nullptr, nullptr, nullptr,
-                                                      (const T*)u, (const T*)dnu, (const C*)b.tw,
-                                                      (C*)b.work);
-      });
+      if constexpr (kLds)
+        gp_cols_lds<T, N, 1><<<lds_tiles<1>(g.S), GNT, 0, s>>>(
+            g, nullptr, nullptr, nullptr, nullptr, (const T*)u, (const T*)dnu, (const C*)b.tw,
+            (C*)b.work);
+      else
+        with_tile(g.S, [&](auto wide, dim3 grid, int threads) {
+          constexpr bool W = decltype(wide)::value;
+          if (g.ucomplex && g.uplanes == 1)
+            gp_cols<T, N, 2, W><<<grid, threads, 0, s>>>(g, nullptr, nullptr, nullptr, nullptr,
+                                                        (const T*)u, nullptr, (const C*)b.tw,
+                                                        (C*)b.work);
+          else
+            gp_cols<T, N, 1, W><<<grid, threads, 0, s>>>(g, nullptr, nullptr, nullptr, nullptr,
+                                                        (const T*)u, (const T*)dnu,
+                                                        (const C*)b.tw, (C*)b.work);
+        });
     }
     if (hy.g_amp_ref) {
       TimedLaunch _t("gp_rows_adj_hyper", s);

@@ -270,32 +270,14 @@ __device__ __forceinline__ void share_packed(cplx<T>* buf, typename FL::Regs& la
   __syncthreads();
 }
 
-// Threads per work-group of the column pass over V columns (register_threads):
-// at most 32 values per thread in FP32; in FP64 one butterfly per thread.
-// With 256 threads whatever the length, a stage of L/R butterflies per column
-// that do not divide by 256 gave some threads two butterflies' registers and
-// left the others idle: at L = 324 (18 x 18, 288 butterflies of 18 points)
-// 177 VGPRs and 2 waves per SIMD against 96 and 5 at 320 threads; in FP64 most
-// lengths ran half empty (measured at 1024^2 x 4E, L = 432 in fold mode,
-// forward / adjoint: 448 / 414 -> 301 / 272 us; L = 512: 603 / 617 -> 328 /
-// 329 us; L = 320 at 512^2: 43 / 43 -> 36 / 33 us).
+// Threads per work-group of the FP64 column pass over V columns
+// (register_threads).  With 256 threads whatever the
+// length most lengths ran half empty (measured at 1024^2 x 4E, forward /
+// adjoint: L = 432 in fold mode 448 / 414 -> 301 / 272 us; L = 512: 603 / 617 ->
+// 328 / 329 us; L = 320 at 512^2: 43 / 43 -> 36 / 33 us).
 template <typename T, int L, int V>
 struct ColThreads {
-  static constexpr int NT = register_threads(L, V, sizeof(T) == 4 ? 32 : 0);
-};
-
-// Exchanges between the stages: complex values, or one component at a time
-// (exchange_split) in FP32 at L = 192, 324 and 432, where the complex tile's
-// LDS and not the registers would bound the resident work-groups.  Measured
-// at 1024^2 x 4E, forward / adjoint, complex against split: L = 324 127 / 108
-// against 107 / 91 us, L = 432 (fold mode) 205 / 162 against 162 / 140 us,
-// L = 192 at 512^2 x 3E 22 / 20 against 17.5 / 16.7 us; elsewhere the two
-// barriers more cost as much as they give (L = 384 82 / 65 against 84 / 67 us,
-// L = 512 133 / 122 against 138 / 127 us, L = 224 at 768^2 52 / 42 against
-// 53 / 43 us, FP64 equal).
-template <typename T, int L>
-struct ColSplit {
-  static constexpr bool value = sizeof(T) == 4 && (L == 192 || L == 324 || L == 432);
+  static constexpr int NT = register_threads(L, V);
 };
 
 // 1-D grid over (sample, column tile, patch, z) with the sample fastest;
@@ -303,7 +285,7 @@ struct ColSplit {
 // remapped so that consecutive items run on one XCD: the S samples of a
 // tile follow each other there and read its kernel-spectrum tile from that
 // XCD's L2 after the first.
-// VC columns per work-group: Tile<T, L>::V, or a half or quarter of it for
+// VC columns per work-group: ColTile<T, L>::V, or a half or quarter of it for
 // geometries with too few tiles to fill the chip (chosen by the autotuner).
 // Every column runs the same butterflies whatever VC is; the instantiations
 // differ only in how the compiler contracts multiply-adds, so results agree
@@ -314,9 +296,11 @@ struct ColSplit {
 // Signal modes read the shared row spectra of lp_rows (R1[(job * n + iy) *
 // H + image row]); the patches of one patch column that share rows (two
 // forward, about L / d in the adjoint) run close together on one XCD (the
-// grid order below) and meet them in its L2.  The forward multiplies each
-// window row by its tent weight on load, through a zero-reading gather so
-// that the multiply does not pull each load into a branch of its own.
+// grid order below) and meet them in its L2.  Rows that do not exist read zero
+// and are not stored by the range check of their buffer resource (RowAccess);
+// the forward multiplies its rows by their tent weights, read from LDS, once
+// all loads are issued.
+// FP64 only: lp_cols_f32 is the FP32 pass.
 template <typename T, int L, int MODE, int VC = ColTile<T, L>::V, bool FOLD = false>
 __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g, const cplx<T>* __restrict__ R1,
                                               const cplx<T>* __restrict__ KT,
@@ -325,14 +309,13 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
                                               cplx<T>* __restrict__ KB, NllFinal fin) {
   constexpr int V = VC;
   constexpr int NT = ColThreads<T, L, VC>::NT;
-  constexpr bool SPLIT = ColSplit<T, L>::value;
-  constexpr int VS = SPLIT ? split_stride(L, V, (int)sizeof(T)) : lds_stride(L, V);
+  constexpr int VS = lds_stride(L, V);
   constexpr int LH = L / 2;
   constexpr int L2P = half_stride(L);
   constexpr int NS = plan_stages(L);
   static_assert(NS <= 2, "the column pass runs plans of one or two stages");
-  static_assert(V >= 2, "the exchange buffer also holds one complex column");
-  __shared__ __align__(16) T buf[(SPLIT ? 1 : 2) * V * VS];
+  static_assert(sizeof(T) == 8, "lp_cols_f32 is the FP32 pass");
+  __shared__ __align__(16) T buf[2 * V * VS];
   __shared__ cplx<T> tw[L];
   __shared__ double red[NT / 64];
   __shared__ double total_s;
@@ -462,10 +445,7 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
     store_twiddles();
     tent_rows(v0);
     F0::compute(v0, tw, tid);
-    if constexpr (SPLIT)
-      exchange_split<F0, FL>(buf, v0, last, tid);
-    else
-      exchange_full<F0, FL>(buf, v0, last, tid);
+    exchange_full<F0, FL>(buf, v0, last, tid);
     FL::compute(last, tw, tid);
   }
 
@@ -581,15 +561,301 @@ __global__ __launch_bounds__((ColThreads<T, L, VC>::NT)) void lp_cols(LinGeom g,
     } else {
       typename IL::Regs v;
       __syncthreads();
-      if constexpr (SPLIT)
-        exchange_split<I0, IL>(buf, last, v, tid);
-      else
-        exchange_full<I0, IL>(buf, last, v, tid);
+      exchange_full<I0, IL>(buf, last, v, tid);
       IL::compute(v, tw, tid);
       if constexpr (kFoldOut)
         fold_out(IL{}, v);
       else
         store_tile(IL{}, v);
+    }
+  }
+  if constexpr (MODE == COL_ADJ) {
+    // The first nseg work-groups also finalise the NLL of the forward pass
+    // that wrote the partials (same order as a one-block reduction).
+    if (fin.out && (int)blockIdx.x < fin.nseg) {
+      const double* pp = fin.partial + (int64_t)blockIdx.x * fin.seglen;
+      double acc = 0.0, nb = 0.0;
+      for (int64_t k = tid; k < fin.seglen; k += NT) acc += pp[k];
+      acc = block_sum<NT>(acc, red);
+      if (fin.report) {
+        const double* pb = pp + (int64_t)fin.nseg * fin.seglen;
+        for (int64_t k = tid; k < fin.seglen; k += NT) nb += pb[k];
+        nb = block_sum<NT>(nb, red);
+      }
+      if (tid == 0) {
+        fin.out[blockIdx.x] = acc;
+        if (fin.report) {
+          fin.report[blockIdx.x] = acc;
+          fin.report[fin.report_n + blockIdx.x] = nb;
+        }
+      }
+    }
+  }
+}
+
+// The FP32 column pass: the work and the arguments of lp_cols with 256 threads
+// and a tile of up to 52 KiB at every length, branches for the rows that do not
+// exist and complex exchanges.  Which product of a sum is rounded before it is
+// contracted to a multiply-add depends on the instructions around a butterfly,
+// so the shape of this kernel is the last bit of the FP32 operator, and the
+// conjugate-gradient solvers amplify that bit: with FP32 in lp_cols a product
+// of the metric moved by 9e-8, and eight steps on a stiff observation by up to
+// 4e-2 of the solution (one right-hand side in ten by more than 2e-5).  In FP64
+// the same steps move by 5e-13 at most over 120 right-hand sides.
+// test_gpu_solve_bits.py holds recorded solutions; tent weights from LDS, the
+// tile loaded before the spectrum and the index split by reciprocals were tried
+// here, and each changes the bits at some lengths.  us forward / adjoint, here
+// against lp_cols: L = 384, 1024^2 x 4E 78 / 66 (79 / 63); L = 324, 1024^2 x 3E x 7
+// modules 744 / 616 (494 / 455; 186 VGPRs, two waves per SIMD, and three by
+// launch bounds spill and are slower); L = 432 in fold mode 53 / 53 (48 / 39); L =
+// 192, 512^2 x 4 samples 19 / 17.
+template <int L, int MODE, int VC = ColTile<float, L>::V, bool FOLD = false>
+__global__ __launch_bounds__(NT) void lp_cols_f32(LinGeom g, const cplx<float>* __restrict__ R1,
+                                                  const cplx<float>* __restrict__ KT,
+                                                  const cplx<float>* __restrict__ twg,
+                                                  cplx<float>* __restrict__ out,
+                                                  cplx<float>* __restrict__ KB, NllFinal fin) {
+  using T = float;
+  constexpr int V = VC;
+  constexpr int VS = lds_stride(L, V);
+  constexpr int LH = L / 2;
+  constexpr int L2P = half_stride(L);
+  constexpr int NS = plan_stages(L);
+  static_assert(NS <= 2, "the column pass runs plans of one or two stages");
+  __shared__ cplx<T> buf[V * VS];
+  __shared__ cplx<T> tw[L];
+  __shared__ double red[NT / 64];
+  __shared__ double total_s;
+  const int tid = threadIdx.x;
+  constexpr int NTILE = (LH + V - 1) / V;
+  const int nsmp = (MODE == COL_KERNEL) ? 1 : g.S;
+  int item = xcd_tile(blockIdx.x, gridDim.x);
+  const int smp = item % nsmp;
+  item /= nsmp;
+  const int k0 = (item % NTILE) * V;
+  item /= NTILE;
+  const int p = item % g.P;
+  const int z = item / g.P;
+
+  int64_t idx, spec;
+  if constexpr (MODE == COL_KERNEL) {
+    const int mod = z / g.Ek, ek = z - mod * g.Ek;
+    spec = ((int64_t)mod * g.P + p) * g.Ek + ek;
+    idx = spec;
+  } else {
+    idx = (int64_t)(smp * g.J + z) * g.P + p;
+    spec = spec_index(g, z, p);
+  }
+  const int lw = FOLD ? g.Lw : L;  // window rows of the cotangent / output
+  const cplx<T>* in;
+  if constexpr (MODE == COL_KERNEL)
+    in = R1 + idx * L2P * g.w;
+  else
+    in = R1 + ((int64_t)r1_image(g, smp, z, MODE == COL_FWD) * g.n + p / g.n) * g.H * L2P;
+  const int m = g.mf, w = g.w;
+
+  // Twiddles are fetched into registers now and stored to LDS once the tile
+  // loads are issued: stage 0 needs none, and the barrier after it orders
+  // the stores before their first use.
+  constexpr int TPT = (L + NT - 1) / NT;
+  cplx<T> twr[TPT];
+#pragma unroll
+  for (int u = 0; u < TPT; ++u) {
+    const int e = tid + u * NT;
+    if (e < L) twr[u] = twg[e];
+  }
+  auto store_twiddles = [&]() {
+#pragma unroll
+    for (int u = 0; u < TPT; ++u) {
+      const int e = tid + u * NT;
+      if (e < L) tw[e] = twr[u];
+    }
+  };
+  T factor = T(1);
+  if constexpr (MODE == COL_KERNEL) {
+    double s = 0.0;
+    for (int rr = tid; rr < w; rr += NT) s += (double)in[rr * L2P].re;
+    s = block_sum<NT>(s, red);
+    if (tid == 0) total_s = s;
+    __syncthreads();
+    factor = T(1.0 / (total_s * (double)L * (double)L));
+  }
+
+  // forward stage 0 straight from global memory
+  using F0 = Stage<T, L, false, 0, V, VS, NT>;
+  using FL = Stage<T, L, false, NS - 1, V, VS, NT>;
+  typename FL::Regs last;
+  // The kernel spectrum of this tile is loaded first: its latency then
+  // overlaps the forward stages instead of stalling the multiply.
+  typename FL::Regs kreg;
+  if constexpr (MODE != COL_KERNEL) {
+    const cplx<T>* ks = KT + spec * L2P * L;
+    FL::gather(kreg, tid, [&](int vec, int pos) -> cplx<T> {
+      const int k = k0 + vec;
+      return k < LH ? ks[pos * L2P + k] : cplx<T>{T(0), T(0)};
+    });
+  }
+  // Image row of window row 0: the adjoint's input rows outside the image
+  // are zero and were never stored; the forward's output rows there are
+  // never read.
+  const int row0 = start_x(g, p % g.n) - g.h - g.m;
+  const Gather gin = make_gather(in, MODE == COL_FWD ? (int64_t)g.H * L2P : 0);
+  const double tstep = tent_step(g.d);
+  auto load_col = [&](int vec, int pos) -> cplx<T> {
+    const int k = k0 + vec;
+    const cplx<T> zero = {T(0), T(0)};
+    if constexpr (MODE == COL_ADJ) {
+      if (k >= LH) return zero;
+      const int ir = row0 + cot_col<FOLD>(g, pos);
+      return (ir >= 0 && ir < g.H) ? ld_stream(&in[ir * L2P + k]) : zero;
+    } else if constexpr (MODE == COL_FWD) {
+      // the tent weight is applied after all loads are issued (tent_rows):
+      // a multiply here would make each task group wait for its loads
+      // before the next group's are issued
+      const int rr = pos - m;
+      const int ir = row0 + g.m + rr;
+      const bool ok = k < LH && rr >= 0 && rr < w && ir >= 0 && ir < g.H;
+      return gather_load<cplx<T>>(gin, gather_off<cplx<T>>(gin, ok, ir * L2P + k));
+    } else {
+      if (k >= LH) return zero;
+      const int rr = pos - m;
+      return (rr >= 0 && rr < w) ? ld_stream(&in[rr * L2P + k]) : zero;
+    }
+  };
+  // forward: window row pos - m carries its tent weight
+  auto tent_rows = [&](typename F0::Regs& regs) {
+    if constexpr (MODE == COL_FWD)
+      F0::for_each(regs, tid, [&](int, int pos, cplx<T>& val) {
+        val = cscale(val, tent_weight<T>(g.d, tstep, pos - m));
+      });
+  };
+  static_assert(F0::Ns == 1, "the first stage takes no twiddles");
+  if constexpr (NS == 1) {
+    F0::gather(last, tid, load_col);
+    store_twiddles();
+    tent_rows(last);
+    __syncthreads();
+    F0::compute(last, tw, tid);
+  } else {
+    typename F0::Regs v0;
+    F0::gather(v0, tid, load_col);
+    store_twiddles();
+    tent_rows(v0);
+    F0::compute(v0, tw, tid);
+    F0::scatter_lds(buf, v0, tid);
+    __syncthreads();
+    FL::gather_lds(buf, last, tid);
+    FL::compute(last, tw, tid);
+  }
+
+  if (k0 == 0) share_packed<FL, T, L>(buf, last, tid);
+  if constexpr (MODE == COL_KERNEL) {
+    cplx<T>* kt = out + spec * L2P * L;
+    FL::emit(last, tid, [&](int vec, int pos, cplx<T> val) {
+      const int k = k0 + vec;
+      if (k >= LH) return;
+      if (k == 0) {
+        // K0 = (P + conj P-)/2, KN = (P - conj P-)/(2i), each with its
+        // ifftshift sign (-1)^(f + k) and the normalisation.
+        const cplx<T> pm = buf[pos == 0 ? 0 : L - pos];
+        const T s0 = (pos & 1) ? -factor : factor;
+        const T sn = ((pos + LH) & 1) ? -factor : factor;
+        const cplx<T> k0v = {T(0.5) * s0 * (val.re + pm.re), T(0.5) * s0 * (val.im - pm.im)};
+        const cplx<T> knv = {T(0.5) * sn * (val.im + pm.im), T(0.5) * sn * (pm.re - val.re)};
+        kt[pos * L2P] = {T(0.5) * (k0v.re + knv.re), T(0.5) * (k0v.im + knv.im)};
+        KB[spec * L + pos] = {T(0.5) * (k0v.re - knv.re), T(0.5) * (k0v.im - knv.im)};
+      } else {
+        const T sgn = ((k + pos) & 1) ? -factor : factor;
+        kt[pos * L2P + k] = cscale(val, sgn);
+      }
+    });
+    return;
+  } else {
+#pragma unroll
+    for (int b = 0; b < FL::BPT; ++b)
+#pragma unroll
+      for (int t = 0; t < FL::R; ++t)
+        last[b][t] = (MODE == COL_ADJ) ? cmulc(last[b][t], kreg[b][t]) : cmul(last[b][t], kreg[b][t]);
+    if (k0 == 0) {
+      // Packed column: alpha P is done above; add beta conj(P[-f]) (the
+      // conjugated factor for the adjoint).  buf holds the raw P.
+#pragma unroll
+      for (int b = 0; b < FL::BPT; ++b) {
+        int vec, j;
+        if (FL::task(tid, b, vec, j) && vec == 0) {
+#pragma unroll
+          for (int t = 0; t < FL::R; ++t) {
+            const int pos = j + t * FL::NB;
+            const cplx<T> pm = buf[pos == 0 ? 0 : L - pos];
+            const cplx<T> pc = {pm.re, -pm.im};
+            const cplx<T> be = KB[spec * L + pos];
+            last[b][t] = cadd(last[b][t], (MODE == COL_ADJ) ? cmulc(pc, be) : cmul(pc, be));
+          }
+        }
+      }
+    }
+    using I0 = Stage<T, L, true, 0, V, VS, NT>;
+    using IL = Stage<T, L, true, NS - 1, V, VS, NT>;
+    static_assert(I0::R == FL::R && I0::BPT == FL::BPT, "shared register layout");
+    I0::compute(last, tw, tid);
+    cplx<T>* o = out + idx * L2P * (MODE == COL_ADJ ? w : lw);
+    auto store = [&](int vec, int pos, cplx<T> val) {
+      const int k = k0 + vec;
+      if (k >= LH) return;
+      if constexpr (MODE == COL_ADJ) {
+        const int r = pos - m;
+        if (r >= 0 && r < w) st_stream(&o[r * L2P + k], val);
+      } else {
+        // Output rows that fall outside the image are never read by the
+        // overlap pass (it gathers image rows only): not stored.
+        const int ir = row0 + pos;
+        if (ir >= 0 && ir < g.H) st_stream(&o[pos * L2P + k], val);
+      }
+    };
+    // Fold mode, forward: the transformed columns go to LDS, and output row
+    // q of the Lw window sums frame positions c, c + Lw and c - Lw, c = q +
+    // mf - m (in [0, L) because L >= Lw); rows outside the image are skipped
+    // as above.
+    auto to_lds = [&](int vec, int pos, cplx<T> val) { buf[vec * VS + pos] = val; };
+    auto fold_out = [&]() {
+      __syncthreads();
+      const int off = g.mf - g.m;
+      for (int e = tid; e < V * lw; e += NT) {
+        const int vec = e & (V - 1), q = e / V;
+        const int k = k0 + vec;
+        const int ir = row0 + q;
+        if (k >= LH || ir < 0 || ir >= g.H) continue;
+        const int c = q + off;
+        const cplx<T>* col = buf + vec * VS;
+        cplx<T> acc = col[c];
+        if (c + lw < L) acc = cadd(acc, col[c + lw]);
+        if (c >= lw) acc = cadd(acc, col[c - lw]);
+        st_stream(&o[q * L2P + k], acc);
+      }
+    };
+    constexpr bool kFoldOut = FOLD && MODE == COL_FWD;
+    if constexpr (NS == 1) {
+      if constexpr (kFoldOut) {
+        __syncthreads();
+        I0::emit(last, tid, to_lds);
+        fold_out();
+      } else {
+        I0::emit(last, tid, store);
+      }
+    } else {
+      __syncthreads();
+      I0::scatter_lds(buf, last, tid);
+      __syncthreads();
+      typename IL::Regs v;
+      IL::gather_lds(buf, v, tid);
+      IL::compute(v, tw, tid);
+      if constexpr (kFoldOut) {
+        __syncthreads();
+        IL::emit(v, tid, to_lds);
+        fold_out();
+      } else {
+        IL::emit(v, tid, store);
+      }
     }
   }
   if constexpr (MODE == COL_ADJ) {
@@ -685,6 +951,9 @@ __device__ __forceinline__ void sum_first_columns(T (&acc)[JPT], const T* buf, c
     iy[t] = first_cover(C + t * NTO, len, g.d, rd);
     c[t] = C + t * NTO - iy[t] * g.d;
   }
+  T sum[N];
+#pragma unroll
+  for (int t = 0; t < N; ++t) sum[t] = T(0);
 #pragma unroll 1
   for (int k = 0; k < steps; ++k) {
 #pragma unroll
@@ -692,12 +961,14 @@ __device__ __forceinline__ void sum_first_columns(T (&acc)[JPT], const T* buf, c
       const int cc = c[t] + (iy[t] == last ? ahead : 0);
       const int v = (iy[t] >> 1) - q0;
       const bool ok = iy[t] <= last && (unsigned)cc < (unsigned)len && (unsigned)v < (unsigned)V;
-      const T x = value(buf + (ok ? 2 * v * VS + (iy[t] & 1) : 0), ok ? cc : 0);
-      acc[t] += ok ? x : T(0);
+      const T x = value(buf + (ok ? 2 * v * VS + (iy[t] & 1) : 0), ok ? cc : 0, sum[t]);
+      sum[t] = ok ? x : sum[t];
       ++iy[t];
       c[t] -= g.d;
     }
   }
+#pragma unroll
+  for (int t = 0; t < N; ++t) acc[t] += sum[t];
 }
 // The first N of a thread's columns lie inside the image: grids of at most one
 // or two times NTO columns skip the others (256^2, a metric of 32 tangents:
@@ -895,15 +1166,15 @@ __global__ __launch_bounds__(NTO) void lp_fwd_out(LinGeom g, const cplx<T>* __re
     __syncthreads();
     fft_lds<T, L, V, VS, NTO, true, kFewVectorPlan<L, V, NTO>>(buf, tw, tid);
     sum_columns<T, V, VS>(acc, reinterpret_cast<const T*>(buf), g, lw, tid + g.h + g.m, q0, steps,
-                          rd, [&](const T* col, int c) {
+                          rd, [&](const T* col, int c, T s) {
                             if constexpr (FOLD) {
                               const int cf = c - g.m + g.mf;
                               T z = col[2 * cf];
                               if (cf + lw < L) z += col[2 * (cf + lw)];
                               if (cf >= lw) z += col[2 * (cf - lw)];
-                              return z;
+                              return s + z;
                             } else {
-                              return col[2 * c];
+                              return s + col[2 * c];
                             }
                           });
     __syncthreads();
@@ -1073,7 +1344,7 @@ __global__ __launch_bounds__(NTO) void lp_adj_out(LinGeom g, const cplx<T>* __re
     fft_lds<T, L, V, VS, NTO, true, kFewVectorPlan<L, V, NTO>>(buf, tw, tid);
     sum_columns<T, V, VS>(tmp, reinterpret_cast<const T*>(buf) + 2 * g.mf, g, g.w, tid + g.h, q0,
                           steps, rd,
-                          [&](const T* col, int c) { return tent_s[c] * col[2 * c]; });
+                          [&](const T* col, int c, T s) { return fma(tent_s[c], col[2 * c], s); });
     __syncthreads();
   };
   for (int job = jb; job < je; job += jstep) {
@@ -1168,10 +1439,20 @@ template <typename T, int L>
 struct LinOps {
   static constexpr int V = ColTile<T, L>::V;
   static constexpr int VR = RowTile<T, L>::V;
-  template <int VC>
-  static constexpr int kColThreads = ColThreads<T, L, VC>::NT;
   static constexpr int LH = L / 2;
   using C = cplx<T>;
+
+  // One column pass over gc work-groups of VC columns, in the kernel of the type.
+  template <int MODE, int VC, bool FOLD>
+  static void cols(int gc, const LinGeom& g, const void* in, const LinBuffers& b, void* out,
+                   NllFinal fin, hipStream_t s) {
+    if constexpr (std::is_same<T, float>::value)
+      lp_cols_f32<L, MODE, VC, FOLD><<<gc, NT, 0, s>>>(
+          g, (const C*)in, (const C*)b.KT, (const C*)b.tw, (C*)out, (C*)b.KB, fin);
+    else
+      lp_cols<T, L, MODE, VC, FOLD><<<gc, ColThreads<T, L, VC>::NT, 0, s>>>(
+          g, (const C*)in, (const C*)b.KT, (const C*)b.tw, (C*)out, (C*)b.KB, fin);
+  }
 
   static int prepare(const LinGeom& g, const LinBuffers& b, const void* kernel, int layout,
                      hipStream_t s) {
@@ -1191,8 +1472,7 @@ struct LinOps {
     const int gc = (LH + V - 1) / V * g.P * g.M * g.Ek;
     {
       TimedLaunch _t("lp_cols_kernel", s);
-      lp_cols<T, L, COL_KERNEL><<<gc, kColThreads<V>, 0, s>>>(g, (const C*)b.R1, nullptr, (const C*)b.tw,
-                                                  (C*)b.KT, (C*)b.KB, NllFinal{});
+      cols<COL_KERNEL, V, false>(gc, g, b.R1, b, b.KT, NllFinal{}, s);
     }
     return launch_status("linpatch_prepare");
   }
@@ -1229,9 +1509,7 @@ struct LinOps {
       with_cols(g, b, [&](auto vc) {
         constexpr int VC = decltype(vc)::value;
         const int gc = g.S * ((LH + VC - 1) / VC) * g.P * g.J;
-        lp_cols<T, L, COL_FWD, VC, FOLD><<<gc, kColThreads<VC>, 0, s>>>(g, (const C*)b.R1, (const C*)b.KT,
-                                                           (const C*)b.tw, (C*)b.R2, (C*)b.KB,
-                                                           NllFinal{});
+        cols<COL_FWD, VC, FOLD>(gc, g, b.R1, b, b.R2, NllFinal{}, s);
       });
     });
     return kOk;
@@ -1261,9 +1539,7 @@ struct LinOps {
       with_cols(g, b, [&](auto vc) {
         constexpr int VC = decltype(vc)::value;
         const int gc = g.S * ((LH + VC - 1) / VC) * g.P * g.J;
-        lp_cols<T, L, COL_ADJ, VC, FOLD><<<gc, kColThreads<VC>, 0, s>>>(g, (const C*)b.R1, (const C*)b.KT,
-                                                           (const C*)b.tw, (C*)b.R2, (C*)b.KB,
-                                                           fin);
+        cols<COL_ADJ, VC, FOLD>(gc, g, b.R1, b, b.R2, fin, s);
       });
     });
     return st;
