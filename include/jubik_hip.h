@@ -322,7 +322,10 @@ int jubik_model_check_domain(jubik_model* model, int64_t* counts, void* stream);
  * kernels write the S NLL values and the counts of the domain check to
  * page-locked host memory of the model, too.  Synchronises ``stream``, writes
  * nll[0 .. S) and counts[0 .. S) (each may be NULL) and returns JUBIK_EDOMAIN
- * as jubik_model_check_domain does. */
+ * as jubik_model_check_domain does.  S is the number of samples of the last
+ * evaluation, by a call or by the launch of a graph (capturing one evaluates
+ * nothing): arrays of max_samples elements hold any result.  JUBIK_ENOTREADY
+ * before the first evaluation. */
 int jubik_model_result(jubik_model* model, double* nll, int64_t* counts, void* stream);
 /* The sampled KL of optimize_kl (demos/x-ray-imaging.py:404-430) at the mean
  * xbar (N x N) for S offsets delta (S x N x N): positions pos[s] = xbar +

@@ -229,7 +229,7 @@ struct jubik_model {
   // host, 2 x max_samples + 1 doubles: NLL and lam <= 0 counts of the last
   // evaluation, and the sum of squared positions of the last sampled KL
   void* report = nullptr;
-  int last_S = 0;           // samples of the last gradient evaluation
+  int last_S = 0;           // samples of the last gradient evaluation (0: none, or it failed)
   int batch_S = 0;          // samples of the last batched gradient (slots 1 .. S)
   void* cg_vec = nullptr;   // solver vectors r, p, Ap, Mv: 4 x max_samples x 2 x N^2
   void* cg_work = nullptr;  // solver scalars and partial sums (doubles)
@@ -299,7 +299,12 @@ static hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 struct jubik_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  std::vector<jubik_model*> points;  // models whose single evaluation sets the base point
+  // gradient evaluations that a launch repeats: samples, and their first slot
+  struct Evaluation {
+    jubik_model* model;
+    int S, slot0;
+  };
+  std::vector<Evaluation> evals;
   int device = 0;
 };
 
@@ -1022,6 +1027,7 @@ int jubik_model_create_batched(jubik_model** model, jubik_gp* gp, jubik_linpatch
   if (!st) st = dev_alloc(&m->resid, img * g.J * S * es, "residual");
   if (!st) st = dev_alloc(&m->partial, 2 * (size_t)g.J * g.H * S * sizeof(double), "NLL partials");
   if (!st) st = host_alloc(&m->report, (2 * S + 1) * sizeof(double), "evaluation report");
+  if (!st) std::memset(m->report, 0, (2 * S + 1) * sizeof(double));
   // GP cotangent: E real planes per sample, or one complex plane (energies
   // folded in) per sample
   if (!st) st = dev_alloc(&m->u, img * std::max(g.E, 2) * S * es, "GP cotangent planes");
@@ -1061,8 +1067,19 @@ int jubik_model_set_data(jubik_model* model, const void* exposure, const int32_t
 
 namespace {
 
+// What the host knows of the model once S evaluations into the slots slot0 ..
+// slot0 + S - 1 are enqueued, by a call or by the launch of a graph (capturing
+// one evaluates nothing).
+void note_evaluation(jubik_model* model, int S, int slot0) {
+  model->last_S = S;
+  model->geo_ready = false;  // slots 0 / 1 changed
+  if (slot0 == 0) model->have_point = true;
+  if (slot0 == 1) model->batch_S = S;
+}
+
 // S gradient evaluations at the positions xi[s]; sky and lam go to slots
-// slot0 .. slot0 + S - 1, nll[s] is the NLL of position s.
+// slot0 .. slot0 + S - 1, nll[s] is the NLL of position s.  Changes no state
+// of the model on the host (see model_evaluate and jubik_graph_launch).
 // With point sources (xi_ps set; the model's point-source prior) the PSF
 // sees the diffuse sky plus p_e = I(xi_ps) exp(alpha dnu_e), and g_ps,
 // g_ps_alpha receive the gradients with respect to xi_ps and xi_ps_alpha.
@@ -1079,7 +1096,6 @@ int model_grad(jubik_model* model, int S, int slot0, const void* amp_ref, const 
                PsArgs pa = PsArgs{}) {
   jubik_linpatch* lp = model->lp;
   jubik_gp* gp = model->gp;
-  model->geo_ready = false;  // slots 0 / 1 change
   GpGeom gg = gp->g;
   gg.zm = zm;
   gg.mu = mu;
@@ -1114,8 +1130,6 @@ int model_grad(jubik_model* model, int S, int slot0, const void* amp_ref, const 
   fin.out = nll;
   fin.report = (double*)model->report;
   fin.report_n = model->max_samples;
-  model->last_S = S;
-  if (slot0 == 1) model->batch_S = S;
   st = linpatch_adjoint_gp(lp->dtype, g, model->lbufs(), model->resid, model->pixel_area, sky,
                            gp->g.has_alpha ? dnu : nullptr, model->u, s, fin,
                            ps ? model->ct : nullptr);
@@ -1130,6 +1144,21 @@ int model_grad(jubik_model* model, int S, int slot0, const void* amp_ref, const 
   return ps_grad(lp->dtype, model->ps, S, g.E, npix, model->ct, model->psw,
                  gp->g.has_alpha ? dnu : nullptr, pa.g_xi, gp->g.has_alpha ? pa.g_xa : nullptr,
                  s);
+}
+
+// model_grad now: a failed one leaves neither results nor positions.
+int model_evaluate(jubik_model* model, int S, int slot0, const void* amp_ref,
+                   const void* amp_alpha, const void* xi_ref, const void* xi_alpha, double zm,
+                   double mu, const void* dnu, double* nll, void* g_ref, void* g_alpha,
+                   hipStream_t s, GpHyper hy = GpHyper{}, PsArgs pa = PsArgs{}) {
+  model->last_S = 0;
+  model->geo_ready = false;
+  if (slot0 == 0) model->have_point = false;
+  if (slot0 == 1) model->batch_S = 0;
+  const int st = model_grad(model, S, slot0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu,
+                            nll, g_ref, g_alpha, s, hy, pa);
+  if (!st) note_evaluation(model, S, slot0);
+  return st;
 }
 
 int check_model(jubik_model* model) {
@@ -1202,11 +1231,8 @@ int jubik_model_grad_points(jubik_model* model, int64_t S, const void* amp_ref,
   pa.g_xa = g_ps_alpha;
   // one position: the metric base point (slot 0); a batch: slots 1 .. S
   const int slot0 = S == 1 ? 0 : 1;
-  if (S == 1) model->have_point = false;
-  st = model_grad(model, (int)S, slot0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll,
-                  g_ref, g_alpha, as_stream(stream), GpHyper{}, pa);
-  if (st == kOk && S == 1) model->have_point = true;
-  return st;
+  return model_evaluate(model, (int)S, slot0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu,
+                        nll, g_ref, g_alpha, as_stream(stream), GpHyper{}, pa);
 }
 
 int jubik_invgamma_prior(int dtype, const void* xi, int64_t n, double a, double q, void* log_i,
@@ -1230,17 +1256,14 @@ int jubik_model_grad_hyper(jubik_model* model, const void* amp_ref, const void* 
     st = fail(kInvalidArgument, "spectral-index inputs are NULL");
   if (st) return st;
   DeviceGuard dg(model->lp->device);
-  model->have_point = false;
   GpHyper hy;
   hy.xi_ref = xi_ref;
   hy.xi_alpha = xi_alpha;
   hy.g_amp_ref = g_amp_ref;
   hy.g_amp_alpha = g_amp_alpha;
   hy.g_off = g_offsets;
-  st = model_grad(model, 1, 0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll, g_ref,
-                  g_alpha, as_stream(stream), hy);
-  if (st == kOk) model->have_point = true;
-  return st;
+  return model_evaluate(model, 1, 0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll,
+                        g_ref, g_alpha, as_stream(stream), hy);
 }
 
 int jubik_model_grad(jubik_model* model, const void* amp_ref, const void* amp_alpha,
@@ -1252,11 +1275,8 @@ int jubik_model_grad(jubik_model* model, const void* amp_ref, const void* amp_al
   if (!st) st = check_alpha(model, amp_alpha, xi_alpha, g_alpha, dnu);
   if (st) return st;
   DeviceGuard dg(model->lp->device);
-  model->have_point = false;
-  st = model_grad(model, 1, 0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll, g_ref,
-                  g_alpha, as_stream(stream));
-  if (st == kOk) model->have_point = true;
-  return st;
+  return model_evaluate(model, 1, 0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll,
+                        g_ref, g_alpha, as_stream(stream));
 }
 
 int jubik_model_grad_batch(jubik_model* model, int64_t S, const void* amp_ref,
@@ -1273,8 +1293,8 @@ int jubik_model_grad_batch(jubik_model* model, int64_t S, const void* amp_ref,
   if (!st) st = check_alpha(model, amp_alpha, xi_alpha, g_alpha, dnu);
   if (st) return st;
   DeviceGuard dg(model->lp->device);
-  return model_grad(model, (int)S, 1, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll,
-                    g_ref, g_alpha, as_stream(stream));
+  return model_evaluate(model, (int)S, 1, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu, nll,
+                        g_ref, g_alpha, as_stream(stream));
 }
 
 int jubik_model_kl_grad(jubik_model* model, int64_t S, const void* amp_ref,
@@ -1308,8 +1328,8 @@ int jubik_model_kl_grad(jubik_model* model, int64_t S, const void* amp_ref,
   st = kl_positions(dtype, (int)S, n, f, (double*)model->partial, max_partial,
                     (double*)model->report + 2 * model->max_samples, s);
   if (!st)
-    st = model_grad(model, (int)S, 1, amp_ref, amp_alpha, pos_ref, pos_alpha, zm, mu, dnu, nll,
-                    gs_ref, gs_alpha, s);
+    st = model_evaluate(model, (int)S, 1, amp_ref, amp_alpha, pos_ref, pos_alpha, zm, mu, dnu,
+                        nll, gs_ref, gs_alpha, s);
   if (!st) st = kl_mean(dtype, (int)S, n, f, s);
   return st;
 }
@@ -1365,7 +1385,7 @@ int jubik_model_grad_graph(jubik_graph** out, jubik_model* model, int64_t S,
   hipStream_t cs = nullptr;
   JUBIK_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
   auto* gr = new jubik_graph();
-  if (S == 0) gr->points.push_back(model);
+  gr->evals.push_back({model, S == 0 ? 1 : (int)S, S == 0 ? 0 : 1});
   gr->device = model->lp->device;
   hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
@@ -1397,7 +1417,7 @@ int jubik_graph_launch(jubik_graph* graph, void* stream) {
   if (!graph || !graph->exec) return fail(kInvalidArgument, "NULL graph");
   DeviceGuard dg(graph->device);
   JUBIK_HIP(hipGraphLaunch(graph->exec, as_stream(stream)));
-  for (jubik_model* m : graph->points) m->have_point = true;
+  for (const auto& e : graph->evals) note_evaluation(e.model, e.S, e.slot0);
   return kOk;
 }
 
@@ -1460,7 +1480,7 @@ int jubik_graph_capture_batch(jubik_graph** out, const jubik_grad_desc* descs, i
       const int wst = jst ? jst : check_hip(hipStreamWaitEvent(cs, ev[i + 1], 0),
                                             "hipStreamWaitEvent");
       if (!cst) cst = wst;
-      if (d.samples == 0) gr->points.push_back(d.model);
+      gr->evals.push_back({d.model, d.samples == 0 ? 1 : (int)d.samples, d.samples == 0 ? 0 : 1});
     }
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(cs, &g);
@@ -1695,12 +1715,11 @@ int jubik_model_geovi_point(jubik_model* model, const void* amp_ref, const void*
   if (!model->geo) st = dev_alloc(&model->geo, 2 * npix * es, "geoVI scalings");
   if (!st && !model->geo_vec) st = dev_alloc(&model->geo_vec, 4 * n * es, "geoVI vectors");
   if (st) return st;
-  model->geo_ready = false;
   // the evaluation at x into slot 1 (its gradient lands in geo_vec and is
   // not used); the base point stays in slot 0
   char* gv = static_cast<char*>(model->geo_vec);
-  st = model_grad(model, 1, 1, amp_ref, amp_alpha, x_ref, x_alpha, zm, mu, dnu, nll, gv,
-                  model->gp->g.has_alpha ? gv + n * es : nullptr, as_stream(stream));
+  st = model_evaluate(model, 1, 1, amp_ref, amp_alpha, x_ref, x_alpha, zm, mu, dnu, nll, gv,
+                      model->gp->g.has_alpha ? gv + n * es : nullptr, as_stream(stream));
   if (!st)
     st = geo_prep(model->lp->dtype, model->counts, model->lam_slot(0), model->lam_slot(1),
                   model->geo, static_cast<char*>(model->geo) + npix * es, npix,

@@ -213,9 +213,9 @@ class XrayModel:
         one synchronisation with the stream (the kernels write them, with the
         counts of ``check_domain``, to host memory).  Raises as
         ``check_domain`` does."""
-        nll = (ctypes.c_double * S)()
+        nll = (ctypes.c_double * max(self.max_samples, 1))()
         _lib.call("jubik_model_result", self._model, nll, None, dev.stream())
-        return nll
+        return nll[:S]
 
     def nll_and_grad(self, xi_ref, xi_alpha=None):
         """(NLL as a Python float, grad_xi_ref, grad_xi_alpha).  Raises
@@ -319,11 +319,11 @@ class XrayModel:
                   dev.ptr(deltas_alpha), s.zm, s.mu, dev.ptr(s.dnu_dev), dev.ptr(nll),
                   dev.ptr(pos[0]), dev.ptr(pos[1]), dev.ptr(gs[0]), dev.ptr(gs[1]),
                   dev.ptr(g_ref), dev.ptr(g_alpha), dev.stream())
-        vals, prior = (ctypes.c_double * S)(), ctypes.c_double()
+        vals, prior = (ctypes.c_double * max(self.max_samples, 1))(), ctypes.c_double()
         _lib.call("jubik_model_kl_result", self._model, vals, ctypes.byref(prior), dev.stream())
         self._batch_S = S
         self._batch_version = s.version
-        return np.array(vals, dtype=np.float64), prior.value, (g_ref, g_alpha)
+        return np.array(vals[:S], dtype=np.float64), prior.value, (g_ref, g_alpha)
 
     def metric_batch(self, v_ref, v_alpha=None):
         """S metric products J^T diag(1/lam) J v at the last gradient position;
