@@ -339,7 +339,8 @@ int jubik_model_kl_grad(jubik_model* model, int64_t S, const void* amp_ref,
                         const void* dnu, double* nll, void* pos_ref, void* pos_alpha,
                         void* gs_ref, void* gs_alpha, void* g_ref, void* g_alpha, void* stream);
 /* jubik_model_result of the last jubik_model_kl_grad, with prior[0] = sum of
- * all squared positions. */
+ * all squared positions.  JUBIK_ENOTREADY when the model's last evaluation was
+ * another one. */
 int jubik_model_kl_result(jubik_model* model, double* nll, double* prior, void* stream);
 /* S gradient evaluations in one pass: xi_ref, xi_alpha, g_ref, g_alpha are
  * (S, N, N) stacks, nll holds S device doubles.  The metric base point is

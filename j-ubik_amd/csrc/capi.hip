@@ -230,6 +230,7 @@ struct jubik_model {
   // evaluation, and the sum of squared positions of the last sampled KL
   void* report = nullptr;
   int last_S = 0;           // samples of the last gradient evaluation (0: none, or it failed)
+  bool kl_ready = false;    // it was a sampled KL: report holds its squared positions
   int batch_S = 0;          // samples of the last batched gradient (slots 1 .. S)
   void* cg_vec = nullptr;   // solver vectors r, p, Ap, Mv: 4 x max_samples x 2 x N^2
   void* cg_work = nullptr;  // solver scalars and partial sums (doubles)
@@ -1072,6 +1073,7 @@ namespace {
 // one evaluates nothing).
 void note_evaluation(jubik_model* model, int S, int slot0) {
   model->last_S = S;
+  model->kl_ready = false;
   model->geo_ready = false;  // slots 0 / 1 changed
   if (slot0 == 0) model->have_point = true;
   if (slot0 == 1) model->batch_S = S;
@@ -1152,7 +1154,7 @@ int model_evaluate(jubik_model* model, int S, int slot0, const void* amp_ref,
                    double mu, const void* dnu, double* nll, void* g_ref, void* g_alpha,
                    hipStream_t s, GpHyper hy = GpHyper{}, PsArgs pa = PsArgs{}) {
   model->last_S = 0;
-  model->geo_ready = false;
+  model->kl_ready = model->geo_ready = false;
   if (slot0 == 0) model->have_point = false;
   if (slot0 == 1) model->batch_S = 0;
   const int st = model_grad(model, S, slot0, amp_ref, amp_alpha, xi_ref, xi_alpha, zm, mu, dnu,
@@ -1331,6 +1333,7 @@ int jubik_model_kl_grad(jubik_model* model, int64_t S, const void* amp_ref,
     st = model_evaluate(model, (int)S, 1, amp_ref, amp_alpha, pos_ref, pos_alpha, zm, mu, dnu,
                         nll, gs_ref, gs_alpha, s);
   if (!st) st = kl_mean(dtype, (int)S, n, f, s);
+  if (!st) model->kl_ready = true;
   return st;
 }
 
@@ -1913,6 +1916,8 @@ int jubik_model_result(jubik_model* model, double* nll, int64_t* counts, void* s
 }
 
 int jubik_model_kl_result(jubik_model* model, double* nll, double* prior, void* stream) {
+  if (model && !model->kl_ready)
+    return fail(kNotReady, "the last evaluation was no sampled KL (call jubik_model_kl_grad)");
   const int st = jubik_model_result(model, nll, nullptr, stream);
   if (!st && prior) *prior = static_cast<const double*>(model->report)[2 * model->max_samples];
   return st;
