@@ -52,12 +52,34 @@ def build_exposure_function(exposures, exposure_cut=None):
     return exposure
 
 
+# Set bits of every byte (numpy counts bits by itself from version 2.0 on only).
+_BITS = np.unpackbits(np.arange(256, dtype=np.uint8)[:, None], axis=1).sum(axis=1)
+
+
+def kept_words(kept):
+    """Bit words of the kept pixels (``kept``: one boolean map per module):
+    an int64 array (2, modules, words) that holds the words, bit b of word k
+    for pixel 64 k + b, and the kept pixels before each word; and the number
+    of kept pixels of every module."""
+    modules = kept.shape[0]
+    per = int(np.prod(kept.shape[1:]))
+    words = np.zeros((2, modules, (per + 63) // 64), dtype=np.int64)
+    bits = words[0].view(np.uint8).reshape(modules, -1)
+    for i in range(modules):
+        packed = np.packbits(kept[i].reshape(-1), bitorder="little")
+        bits[i, :packed.size] = packed
+    upto = np.cumsum(_BITS[bits].reshape(words[0].shape + (8,)).sum(axis=-1), axis=1,
+                     dtype=np.int64)
+    words[1, :, 1:] = upto[:, :-1]
+    return words, (upto[:, -1].tolist() if words.shape[2] else [0] * modules)
+
+
 def build_readout_function(flags, threshold=None, keys=None):
     """jubik/response.py:48-112: returns ``x -> Vector({key_i: x[i][~mask[i]]})``.
 
     ``mask = (flags == 0)`` after zeroing the flags below ``threshold`` in
-    place.  The read-out is a gather by the precomputed C-order indices of
-    the kept pixels of every module.
+    place.  The kept pixels are held as a bit each (``kept_words``) and read out
+    in C order, all modules in one launch.
     """
     if threshold is not None and threshold < 0:
         raise ValueError("threshold should be positive!")
@@ -77,15 +99,7 @@ def build_readout_function(flags, threshold=None, keys=None):
         modules, words), and the number of kept pixels per module."""
         dkey = torch.cuda.current_device()
         if dkey not in word_cache:
-            per = int(np.prod(mask.shape[1:]))
-            nwords = (per + 63) // 64
-            host = np.zeros((2, len(keys), nwords), dtype=np.int64)
-            for i in range(len(keys)):
-                bits = np.packbits(~mask[i].reshape(-1), bitorder="little")
-                host[0, i].view(np.uint8)[:bits.size] = bits
-            kept = np.cumsum(np.bitwise_count(host[0].view(np.uint64)), axis=1, dtype=np.int64)
-            host[1, :, 1:] = kept[:, :-1]
-            counts = kept[:, -1].tolist() if nwords else [0] * len(keys)
+            host, counts = kept_words(~mask[:len(keys)])
             word_cache[dkey] = (torch.as_tensor(host, device="cuda"), counts)
         return word_cache[dkey]
 
