@@ -54,18 +54,26 @@ class Poissonian:
             dt = dev.to_device(d, dtype).reshape(-1)
             if lt.numel() != dt.numel():
                 raise ValueError("lambda and data sizes differ")
+            groups.setdefault(dtype, []).append(len(parts))
             parts.append((lt, dt, torch.empty_like(lt)))
-            groups.setdefault(dtype, []).append(len(parts) - 1)
-        nll = torch.empty(len(parts), dtype=torch.float64, device="cuda")
-        work = torch.empty(len(parts) * (_lib.POISSON_WORK_BYTES // 8), dtype=torch.float64,
-                           device="cuda")
-        order = []  # leaf of every entry of nll
+        words = _lib.POISSON_WORK_BYTES // 8
+        # per leaf its energy, then the work of the reductions
+        buf = torch.empty(len(parts) * (1 + words), dtype=torch.float64, device="cuda")
+        nll = buf[:len(parts)]
+        at, order = buf.data_ptr(), []  # order: leaf of every entry of nll
+        work = ctypes.c_void_p(at + 8 * len(parts))
         for dtype, members in groups.items():
-            lts, dts, gs = zip(*[parts[i] for i in members])
-            sizes = (ctypes.c_int64 * len(members))(*[t.numel() for t in lts])
-            _lib.call("jubik_poisson_nll_grad_segments", dev.code(dtype), len(members),
-                      dev.ptrs(lts), dev.ptrs(dts), sizes, dev.ptr(nll[len(order):]),
-                      dev.ptrs(gs), dev.ptr(work), dev.stream())
+            value = ctypes.c_void_p(at + 8 * len(order))
+            if len(members) == 1:  # needs no host arrays of pointers and sizes
+                lt, dt, g = parts[members[0]]
+                _lib.call("jubik_poisson_nll_grad", dev.code(dtype), dev.ptr(lt), dev.ptr(dt),
+                          lt.numel(), value, dev.ptr(g), work, dev.stream())
+            else:
+                lts, dts, gs = zip(*[parts[i] for i in members])
+                sizes = (ctypes.c_int64 * len(members))(*[t.numel() for t in lts])
+                _lib.call("jubik_poisson_nll_grad_segments", dev.code(dtype), len(members),
+                          dev.ptrs(lts), dev.ptrs(dts), sizes, value, dev.ptrs(gs), work,
+                          dev.stream())
             order += members
         total = 0.0
         for _, value in sorted(zip(order, nll.tolist())):

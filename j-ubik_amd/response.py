@@ -5,6 +5,8 @@ checks, in-place cut of the caller's array, key handling); the closures
 they return run as HIP kernels (broadcast multiply, gather of the kept pixels
 in C order).
 """
+import math
+
 import numpy as np
 import torch
 
@@ -92,16 +94,19 @@ def build_readout_function(flags, threshold=None, keys=None):
     elif len(keys) != flags.shape[0]:
         raise ValueError("length of keys should match the number of flag maps.")
     word_cache = {}
+    pixels = math.prod(mask.shape[1:])
 
     def _words():
         """Kept pixels of the modules that are read out, on the current
-        device: bit words and kept pixels before each word, stacked (2,
-        modules, words), and the number of kept pixels per module."""
+        device: pointers to the bit words and to the kept pixels before each
+        word, and the number of kept pixels per module (and the tensor that
+        the pointers lie in)."""
         dkey = torch.cuda.current_device()
         if dkey not in word_cache:
             host, counts = kept_words(~mask[:len(keys)])
-            word_cache[dkey] = (torch.as_tensor(host, device="cuda"), counts)
-        return word_cache[dkey]
+            words = torch.as_tensor(host, device="cuda")
+            word_cache[dkey] = (dev.ptr(words[0]), dev.ptr(words[1]), counts, words)
+        return word_cache[dkey][:3]
 
     def _apply_readout(x):
         if len(mask.shape) != 4:
@@ -111,15 +116,15 @@ def build_readout_function(flags, threshold=None, keys=None):
         dev.require_device()
         dtype = dev.float_dtype(x)
         xt = dev.to_device(x, dtype)
-        per, pixels = int(np.prod(xt.shape[1:])), int(np.prod(mask.shape[1:]))
+        per = math.prod(xt.shape[1:])
         if xt.shape[0] < len(keys):
             raise IndexError("input has fewer modules than there are keys")
         if per < pixels:
             raise ValueError("input module shape does not match the flags")
-        words, counts = _words()
+        words, before, counts = _words()
         out = [torch.empty(c, dtype=dtype, device="cuda") for c in counts]
-        _lib.call("jubik_readout_gather_words", dev.code(dtype), len(keys), dev.ptr(words[0]),
-                  dev.ptr(words[1]), pixels, dev.ptr(xt), per, dev.ptrs(out), dev.stream())
+        _lib.call("jubik_readout_gather_words", dev.code(dtype), len(keys), words, before, pixels,
+                  dev.ptr(xt), per, dev.ptrs(out), dev.stream())
         return Vector({key: dev.like_input(v, x) for key, v in zip(keys, out)})
 
     def _transpose(vec, like_shape=None):
@@ -128,16 +133,15 @@ def build_readout_function(flags, threshold=None, keys=None):
         shape = mask.shape
         first = vec[keys[0]]
         dtype = dev.float_dtype(first)
-        words, counts = _words()
+        words, before, counts = _words()
         vs = [dev.to_device(vec[key], dtype) for key in keys]
         if any(v.numel() < c for v, c in zip(vs, counts)):
             raise ValueError("read-out vectors are shorter than the kept pixels")
         # modules that are not read out stay zero
         new = torch.empty if len(keys) == shape[0] else torch.zeros
         out = new(shape, dtype=dtype, device="cuda")
-        _lib.call("jubik_readout_scatter_words", dev.code(dtype), len(keys), dev.ptr(words[0]),
-                  dev.ptr(words[1]), int(np.prod(shape[1:])), dev.ptrs(vs), dev.ptr(out),
-                  dev.stream())
+        _lib.call("jubik_readout_scatter_words", dev.code(dtype), len(keys), words, before, pixels,
+                  dev.ptrs(vs), dev.ptr(out), dev.stream())
         return dev.like_input(out, first)
 
     _apply_readout.transpose = _transpose
