@@ -253,12 +253,10 @@ constexpr int kOutOfRange = (int)0x80000000;  // lies past every range
 // lie past the range that the hardware checks.  So a column's loads and
 // stores cost one addition each, or none with a constant shift of whole rows
 // inside the range (``step``), where bounds checks and 64-bit addresses
-// took six to eight instructions.  The column passes issue instructions for
-// half their time: at L = 384 the forward went from 2885 to 2053 vector
-// instructions a tile (with the tent weights read from LDS), the adjoint from
-// 2747 to 2023; measured forward / adjoint, 1024^2 x 4E 79 / 68 -> 79 / 63 us,
-// 1024^2 x 3E x 7 modules (L = 324) 523 / 480 -> 494 / 455 us, fold mode at
-// L = 432 53 / 45 -> 48 / 39 us.  Arrays stay below 1 GiB.
+// took six to eight instructions.  Used by the FP64 column pass of the PSF (L =
+// 320 at 512^2 x 2E, with the tent weights read from LDS, forward / adjoint 23 /
+// 22.5 -> 21.5 / 20.5 us) and for the stores of the sky's.  Arrays stay below 1
+// GiB.
 template <typename T, int STRIDE>
 struct RowAccess {
   typedef unsigned int u2 __attribute__((ext_vector_type(2)));

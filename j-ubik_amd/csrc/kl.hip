@@ -3,7 +3,8 @@
 // Both kernels stream: they read and write each array once and are bound by
 // that traffic.  As separate array operations (broadcast add, conversion to
 // double, squares, sums and means) the same results took about 750 us of a
-// 2048^2 x 2-field, 4-sample KL evaluation; fused they take 116 us (0.55 GB).
+// 2048^2 x 2-field, 4-sample KL evaluation; fused they take 114 us (18 passes over
+// a field of 33.6 MB, 0.60 GB).
 #include <algorithm>
 
 #include "kl.hpp"

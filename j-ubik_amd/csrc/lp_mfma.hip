@@ -11,7 +11,7 @@
 // radix-3 step runs in FP32.  The inverse transform is conj(DFT(conj(.)))
 // (unnormalised, like the FFT path; the kernel spectra carry the 1 / L^2).
 //
-// The pass replaces lp_cols<float, 384, COL_FWD / COL_ADJ> outside fold
+// The pass replaces lp_cols_f32<384, COL_FWD / COL_ADJ> outside fold
 // mode: the same inputs, outputs, row skipping, kernel-spectrum multiply
 // (packed DC/Nyquist column included) and NLL finalisation.  A persistent
 // work-group of 8 waves keeps the C and S fragments of rows 0..63 (64 KiB

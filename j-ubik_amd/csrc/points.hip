@@ -8,13 +8,16 @@
 // The inverse-gamma prior maps a standard normal xi to the inverse-gamma
 // variable of shape a and scale q with the same quantile: I = q / y with
 // Q(a, y) = Phi(xi), Q the regularised upper incomplete gamma function (if
-// Y ~ Gamma(a, 1) then P(q / Y <= x) = Q(a, q / x)).  y is found by Newton
+// Y ~ Gamma(a, 1) then P(q / Y <= x) = Q(a, q / x)).  y is found by Halley
 // steps in log y on log P(a, y) = log Phi(-xi) (small y) or log Q(a, y) =
-// log Phi(xi) (large y), started from the Wilson-Hilferty approximation of
-// the Gamma quantile (whose standard normal quantile is exactly -xi) or, for
-// small y or a < 1, from the leading term y^a / Gamma(a + 1) of P.  P and Q
-// come from their power series (y < a + 1) or the continued fraction of Q
-// (modified Lentz), in double precision.  The derivative is closed-form:
+// log Phi(xi) (large y), started for a >= 1 from the Wilson-Hilferty
+// approximation of the Gamma quantile (whose standard normal quantile is
+// exactly -xi) or, for small y, from the leading term y^a / Gamma(a + 1) of P,
+// and for a < 1 from the two-branch approximation of Numerical Recipes (Press
+// et al., 3rd edition 2007, section 6.2.1, which also takes Halley steps).  P and
+// Q come from their power series (y < a + 1) or the continued fraction of Q
+// (modified Lentz); the last steps are in double precision.  The derivative is
+// closed-form:
 //   d log I / d xi = phi(xi) Gamma(a) / (y^a e^-y).
 #include <cmath>
 
